@@ -131,7 +131,6 @@ static int exec_workspace(size_t need, void** out) {
 // 4 K ranges x 1024 x 2560 floats of partial sums; its attention runs on
 // folded 64-row blocks with no workspace); the GPT-2 and 7B workloads need at
 // most 25 MiB.
-#define LBR_SCRATCH_BYTES ((size_t)48 << 20)
 #define LBR_MAX_DEVICES 64
 static __device__ __align__(256) unsigned char scratch[LBR_SCRATCH_BYTES];
 static void* g_scratch_dev[LBR_MAX_DEVICES] = {};
@@ -485,7 +484,7 @@ static void table_tiles(std::vector<Step>& steps, std::vector<char>* tabled) {
         if (!s.name || strncmp(s.name, "gemm_dma_f32", 12) != 0 || !s.i[14] || s.i[3] != 1) continue;
         for (const TunedTile& t : kTunedTiles) {
             if (strcmp(s.name, t.step) != 0 || s.i[0] != t.M || s.i[1] != t.N || s.i[2] != t.K) continue;
-            const int tile = gemm_dma_tile_by_name(t.tile);
+            const int tile = gemm_dma_tile_by_name(s, t.tile);
             Step u = s;
             if (tile < 0 || !gemm_dma_retile(&u, tile) || (t.ks > 0 && !gemm_dma_set_ksplit(&u, t.ks))) continue;
             s = u;

@@ -1763,7 +1763,7 @@ bool lbr_merge_gemm_head_prologue(Step* g, const Step& h, const OpNode* nodes, i
                 if (overlap(r, rng(live_ptr[q], (long long)live_bytes[q]))) return false;
     }
     Step t = *g;
-    if (!gemm_dma_retile(&t, gemm_dma_tile_by_name("64x128"))) return false;
+    if (!gemm_dma_retile(&t, gemm_dma_tile_by_name(t, "64x128"))) return false;
     t.i[18] = parts;
     for (int p = 0; p < 2; ++p) {
         t.i[20 + p] = col[p];

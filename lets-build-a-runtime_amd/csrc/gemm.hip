@@ -8,11 +8,12 @@
 //               reference hard-codes alpha = 1 on this path, executor.c:341/344)
 // op(B) = Bᵀ when trans_b (B stored [N, K], nn.Linear layout) else B ([K, N]).
 //
-// Two kernels: gemm_dma_f32 (below the register-staged one) takes every
-// trans_b GEMM with K a multiple of 32 — all the Linear layers of the
-// workloads — with v_mfma_f32_16x16x4_f32, direct-to-LDS loads and a tile
-// shape chosen per GEMM; gemm_mfma_f32 (v_mfma_f32_32x32x2_f32) takes the
-// rest (B stored [K, N], ragged K, unaligned operands).
+// Three kernels: gemm_dma_f32 (below the register-staged one) takes trans_b GEMMs with K
+// a multiple of 32 — all the Linear layers of the workloads — with
+// v_mfma_f32_16x16x4_f32, direct-to-LDS loads and a tile shape chosen per GEMM; of those,
+// gemm_split_f32 (gemm_split.hip) takes the large ones (use_split) on the bf16 matrix
+// cores; gemm_mfma_f32 (v_mfma_f32_32x32x2_f32) takes the rest (B stored [K, N], ragged
+// K, unaligned operands).
 //
 // gemm_mfma_f32 tiling: a 256-thread workgroup (4 wavefronts, 2×2) owns a 128×128 tile of
 // C; each wavefront owns 64×64 = 2×2 MFMA blocks of 32×32 (64 accumulator
@@ -28,115 +29,97 @@
 // are mapped round-robin over the 8 XCDs by the hardware; the remap below
 // gives each XCD a contiguous range of tiles so neighbouring tiles (which
 // reuse the same A and B panels) hit the same L2.
-#include "lbr_device.h"
+#include "gemm_common.h"
 
+#include <cstdio>
 #include <cstdlib>
 #include <cstring>
+
+// Step::i: [0]=M [1]=N [2]=K [3]=batches [4]=trans_b [5]=fragment-major head splits [6]=has_bias
+//          [7]=sA [8]=sB [9]=sC [10]=ksplit [11]=kchunk [12]=float4 reduce
+//          [13]=1 (takes fused epilogues) [14]=DMA tile + 1 (0: gemm_mfma_f32)
+//          [19..30] head scatter, [31] activation, [32..34] gated pair, [35..37] A in
+//          head layout (see below) ; f[0] = alpha
+GemmArgs gemm_make_args(const Step& s) {
+    GemmArgs g;
+    g.A = (const float*)s.in[0];
+    g.B = (const float*)s.in[1];
+    g.bias = (const float*)s.in[2];
+    g.C = (float*)s.out;
+    g.M = (int)s.i[0];
+    g.N = (int)s.i[1];
+    g.K = (int)s.i[2];
+    g.sA = s.i[7];
+    g.sB = s.i[8];
+    g.sC = s.i[9];
+    g.alpha = s.f[0];
+    g.ksplit = s.i[10] > 1 ? (int)s.i[10] : 1;
+    g.kchunk = g.ksplit > 1 ? (int)s.i[11] : g.K;
+    g.W = (float*)s.ws;
+    // fused epilogue: in[3] = resid (gated pair: the GATED_ACT bias);
+    // i[19] = n_split, i[20..24] = col_begin, in[4..7] = dst, in[8..11] =
+    // split biases, i[25..28] = heads per split, i[29] = hd, i[30] = S,
+    // i[5] = splits stored fragment-major (bit k, set by the plan);
+    // i[31] = act; i[32] = gated F, i[33] = gated act, i[34] = gate half's first column
+    g.gF = (int)s.i[32];
+    g.gact = (int)s.i[33];
+    g.gbase = (int)s.i[34];
+    g.resid = g.gF ? nullptr : (const float*)s.in[3];
+    g.gbias = g.gF ? (const float*)s.in[3] : nullptr;
+    g.n_split = (int)s.i[19];
+    for (int k = 0; k < 5; ++k) g.col_begin[k] = (int)s.i[20 + k];
+    for (int k = 0; k < 4; ++k) {
+        g.dst[k] = (float*)s.in[4 + k];
+        g.sbias[k] = (const float*)s.in[8 + k];
+        g.Hs[k] = (int)s.i[25 + k];
+    }
+    g.hd = (int)s.i[29];
+    g.S = (int)s.i[30];
+    g.frag = (int)s.i[5];
+    // i[18] = head prologue parts (0: none; see lbr_merge_gemm_head_prologue), i[20..23]
+    // = their first columns and heads, i[24] = flags, i[25..26] = RoPE row strides over
+    // b and s, i[30] = S; in[4..5] outputs, in[6..7] norm weights, in[8..9] cos / sin,
+    // in[10..11] biases; f[2..3] eps
+    g.hp_parts = (int)s.i[18];
+    g.hp_flags = (int)s.i[24];
+    g.hp_S = (int)s.i[30];
+    for (int p = 0; p < 2; ++p) {
+        g.hp_col[p] = (int)s.i[20 + p];
+        g.hp_H[p] = (int)s.i[22 + p];
+        g.hp_out[p] = (float*)s.in[4 + p];
+        g.hp_w[p] = (const float*)s.in[6 + p];
+        g.hp_b[p] = (const float*)s.in[10 + p];
+        g.hp_eps[p] = s.f[2 + p];
+    }
+    g.hp_cos = (const float*)s.in[8];
+    g.hp_sin = (const float*)s.in[9];
+    g.hp_tst[0] = s.i[25];
+    g.hp_tst[1] = s.i[26];
+    g.act = (int)s.i[31];
+    // i[35..37] = A in head layout [B, H, S, hd]: H, S, hd (0: row-major A)
+    g.aH = (int)s.i[35];
+    g.aS = (int)s.i[36];
+    g.ahd = (int)s.i[37];
+    // i[15] = norm prologue (LBR_NORM_*), i[38] / i[39] = its weight / bias, f[1] = eps
+    g.nw = (const float*)(uintptr_t)s.i[38];
+    g.nb = (const float*)(uintptr_t)s.i[39];
+    g.neps = s.f[1];
+    // i[16] = norm after the split-K reduce (LBR_NORM_*), i[17] = its form
+    // (16·(1 wave / 2 block per row) + float4 per lane, + 256 when the K split
+    // was made for the norm); in[4] output, in[5]
+    // weight, in[6] LayerNorm bias, f[2] eps (the head-split fields are unused
+    // then: i[19] = 0)
+    g.nt_out = s.i[16] ? (float*)s.in[4] : nullptr;
+    g.nt_w = s.i[16] ? (const float*)s.in[5] : nullptr;
+    g.nt_b = s.i[16] ? (const float*)s.in[6] : nullptr;
+    g.nt_eps = s.f[2];
+    return g;
+}
 
 namespace {
 
 constexpr int BM = 128, BN = 128, BK = 32, LDK = BK + 4;
 constexpr int NT = 256;
-constexpr int N_XCD = 8;
-constexpr int GROUP_M = 8;   // tile rows per L2 group
-
-struct GemmArgs {
-    const float* A;
-    const float* B;
-    float* C;
-    const float* bias;
-    int M, N, K;
-    long long sA, sB, sC;     // batch strides (elements)
-    float alpha;
-    int tiles_m, tiles_n;
-    float* W;                 // split-K partial sums [ksplit][batches][M][N] (ksplit > 1)
-    int ksplit, kchunk;       // number of K ranges, K per range (multiple of BK)
-    // Fused epilogues (set only by the plan's peephole fusion; all null/0 otherwise).
-    const float* resid;       // C += resid (same layout as C): a following same-shape ADD
-    int n_split;              // >0: C columns are scattered as attention heads, see epi_store
-    int col_begin[5];         // split k owns columns [col_begin[k], col_begin[k+1])
-    float* dst[4];            // split k's output, laid out [B, H, S, hd]
-    const float* sbias[4];    // split k's bias row (indexed by column - col_begin[k]) or null
-    int Hs[4], hd, S;         // heads of each split, head dim, rows per batch (M = B·S)
-    int frag;                 // bit k: split k is stored fragment-major (lbr_frag_offset)
-    // Head prologue in the epilogue (lbr_merge_gemm_head_prologue; 64×128 DMA tile, hd =
-    // 128 = TN): C columns [hp_col[p], hp_col[p] + hp_H[p]·128) of part p hold heads of
-    // 128; each tile's C values (+ bias) go round through LDS, get the part's bias,
-    // per-head RMSNorm (weight hp_w[p], eps hp_eps[p]) and rotate-half RoPE (cos/sin row
-    // of token (b, s) at b·hp_tst[0] + s·hp_tst[1]) and are stored as [B, H, S, 128] at
-    // hp_out[p] (C's columns of the parts are not written); hp_flags: 1 norm, 2 RoPE
-    int hp_parts, hp_flags, hp_S;
-    int hp_col[2], hp_H[2];
-    float* hp_out[2];
-    const float* hp_w[2];
-    const float* hp_b[2];
-    float hp_eps[2];
-    const float* hp_cos;
-    const float* hp_sin;
-    long long hp_tst[2];
-    int act;                  // LBR_ACT_*: a following RELU / GELU / SILU applied to C (DMA kernel)
-    // Gated pair (DMA kernel): the GEMM's columns hold a gate half and an up half
-    // of gF columns each; the kernel writes out[m][j] = act(gate[m][j] (+ gbias[j]))·up[m][j]
-    // to C as [M, gF]
-    int gF;                   // 0: off
-    int gbase;                // first column of the gate half (0 or gF; up is the other half)
-    int gact;                 // 0: SiLU, 1: GELU (GATED_ACT extras[1])
-    const float* gbias;       // GATED_ACT bias (applied to gate) or null
-    // A in head layout (DMA kernel): A is stored [B, aH, aS, ahd] and read as the
-    // [B·aS, aH·ahd] matrix its TRANSPOSE(1, 2) would give (aH = 0: A is row-major)
-    int aH, aS, ahd;
-    // Norm prologue (DMA kernel, NORM template argument): A is the input of a
-    // RMSNORM / LAYERNORM over its K columns whose output was this GEMM's A;
-    // nw = weight (γ), nb = LayerNorm bias (β), neps = eps
-    const float* nw;
-    const float* nb;
-    float neps;
-    // Norm after the split-K reduce (lbr_merge_reduce_norm): the reduce, one row
-    // at a time, also normalises C's row into nt_out (RMSNORM / LAYERNORM over
-    // the N columns, weight nt_w, LayerNorm bias nt_b)
-    float* nt_out;
-    const float* nt_w;
-    const float* nt_b;
-    float nt_eps;
-};
-
-// Final store of one C element (row m, column n of batch bz) with the fused
-// epilogues applied in the order the unfused nodes would: v (already
-// alpha-scaled or bias-added) + resid, then the scattered split's bias.
-__device__ __forceinline__ void epi_store(const GemmArgs& g, long long bz, int m, int n, float v) {
-    if (g.resid) v = v + g.resid[bz * g.sC + (long long)m * g.N + n];
-    if (g.n_split == 0) {
-        g.C[bz * g.sC + (long long)m * g.N + n] = v;
-        return;
-    }
-    if (n < g.col_begin[0] || n >= g.col_begin[g.n_split]) return;   // columns no split reads
-    int k = 0;
-    while (k + 1 < g.n_split && n >= g.col_begin[k + 1]) ++k;
-    const int c = n - g.col_begin[k];
-    if (g.sbias[k]) v = v + g.sbias[k][c];
-    const int h = c / g.hd, d = c - h * g.hd;
-    const int b = m / g.S, s = m - b * g.S;
-    const long long head = ((long long)b * g.Hs[k] + h) * g.S * g.hd;
-    g.dst[k][head + (((g.frag >> k) & 1) ? lbr_frag_offset(s, d, g.hd) : (long long)s * g.hd + d)] = v;
-}
-
-__device__ __forceinline__ void tile_coords(const GemmArgs& g, int& tm, int& tn) {
-    // XCD-aware remap: hardware places workgroup id w on XCD w % 8.
-    const int tiles = g.tiles_m * g.tiles_n;
-    int w = blockIdx.x;
-    if (tiles % N_XCD == 0) {
-        const int per = tiles / N_XCD;
-        w = (w % N_XCD) * per + (w / N_XCD);
-    }
-    // grouped ordering: GROUP_M tile-rows advance together along N
-    const int group_size = GROUP_M * g.tiles_n;
-    const int gid = w / group_size;
-    const int first_m = gid * GROUP_M;
-    const int gm = min(g.tiles_m - first_m, GROUP_M);
-    const int in_group = w % group_size;
-    tm = first_m + in_group % gm;
-    tn = in_group / gm;
-}
 
 template <bool TRANS_B, bool VEC>
 __device__ __forceinline__ void load_tiles(const GemmArgs& g, const float* __restrict__ A, const float* __restrict__ B,
@@ -684,9 +667,8 @@ __global__ __launch_bounds__(64 * WGM * WGN, OCC) void gemm_dma_f32(GemmArgs g) 
         __builtin_amdgcn_s_waitcnt(0x3F70);   // no DMA may still target this workgroup's LDS at exit
     }
 
-    const int rq = (lane >> 4) * 4, cl = lane & 15;
-    const int mw = m0 + wm * (TM / WGM), nw = n0 + wn * (TN / WGN);
     if (NORM) {
+        const int rq = (lane >> 4) * 4;
         // whole rows: sum the four kq lanes of each row and column, then take
         // each accumulator row's factors from the lane that holds that row
         const float invK = 1.0f / K;
@@ -729,171 +711,8 @@ __global__ __launch_bounds__(64 * WGM * WGN, OCC) void gemm_dma_f32(GemmArgs g) 
             }
         }
     }
-    if constexpr (TM == 64 && TN == 128 && WGM == 2 && WGN == 2 && !AHEADS && NORM == 0) {
-        int p = -1;
-        for (int q = 0; q < g.hp_parts; ++q)
-            if (n0 >= g.hp_col[q] && n0 < g.hp_col[q] + g.hp_H[q] * TN) p = q;
-        if (p >= 0) {
-            // one head per tile: C (+ bias) through LDS, then each wavefront takes 16 rows,
-            // two a pass, a row over 32 lanes of 4 columns each — the lanes, sums and
-            // partner swaps of head_rows4 at HD = 128, so the values are the same bits
-            constexpr int TS = TN + 4;
-            static_assert(TM * TS <= NS * STAGE, "the tile fits in the stages");
-            __syncthreads();   // every wavefront's last fragment reads are done
-#pragma unroll
-            for (int j = 0; j < FN; ++j) {
-                const int c = wn * (TN / WGN) + j * 16 + cl;
-                const float bv = HAS_BIAS ? g.bias[n0 + c] : 0.f;
-#pragma unroll
-                for (int i = 0; i < FM; ++i)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        lds[(wm * (TM / WGM) + i * 16 + rq + r) * TS + c] =
-                            HAS_BIAS ? (acc[i][j][r] + bv) : g.alpha * acc[i][j][r];
-            }
-            __syncthreads();
-            const int H = g.hp_H[p], h = (n0 - g.hp_col[p]) / TN, S = g.hp_S;
-            const int l = lane & 31, d = 4 * l;
-            const bool norm = g.hp_flags & 1, rope = g.hp_flags & 2;
-            const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
-            const float4 wv = norm ? *reinterpret_cast<const float4*>(g.hp_w[p] + d) : zero;
-            const float* __restrict__ pbias = g.hp_b[p];
-            const float4 pb = pbias ? *reinterpret_cast<const float4*>(pbias + h * TN + d) : zero;
-            const float eps = g.hp_eps[p];
-#pragma unroll 2
-            for (int pass = 0; pass < TM / NW / 2; ++pass) {
-                const int row = wave * (TM / NW) + 2 * pass + (lane >> 5);
-                const int m = m0 + row, mc = min(m, M - 1);
-                const int b = mc / S, s = mc - b * S;
-                const float4 x = *reinterpret_cast<const float4*>(&lds[row * TS + d]);
-                float4 v = x;
-                if (pbias) {
-                    v.x = v.x + pb.x;
-                    v.y = v.y + pb.y;
-                    v.z = v.z + pb.z;
-                    v.w = v.w + pb.w;
-                }
-                float4 c4 = zero, s4 = zero;
-                if (rope) {
-                    const long long t = b * g.hp_tst[0] + s * g.hp_tst[1] + d;
-                    c4 = *reinterpret_cast<const float4*>(g.hp_cos + t);
-                    s4 = *reinterpret_cast<const float4*>(g.hp_sin + t);
-                }
-                const float4 y = lbr_head_row<32, TN>(v, norm, wv, eps, rope, c4, s4, lane);
-                if (m < M)
-                    *reinterpret_cast<float4*>(g.hp_out[p] + (((long long)b * H + h) * S + s) * TN + d) = y;
-            }
-            return;
-        }
-    }
-    if (g.ksplit > 1) {
-        float* __restrict__ Wp = g.W + ((long long)ks * gridDim.z + bz) * (long long)M * N;
-#pragma unroll
-        for (int j = 0; j < FN; ++j) {
-            const int n = nw + j * 16 + cl;
-            if (n >= N) continue;
-#pragma unroll
-            for (int i = 0; i < FM; ++i)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int m = mw + i * 16 + rq + r;
-                    if (m < M) Wp[(long long)m * N + n] = acc[i][j][r];
-                }
-        }
-        return;
-    }
-    if (g.n_split) {
-        // head scatter: the column fixes split, head, d and split bias; the
-        // row fixes (b, s) = divmod(m, S), stepped from each 4-row group's first row
-#pragma unroll
-        for (int j = 0; j < FN; ++j) {
-            const int n = nw + j * 16 + cl;
-            if (n >= N || n < g.col_begin[0] || n >= g.col_begin[g.n_split]) continue;
-            int k = 0;
-            while (k + 1 < g.n_split && n >= g.col_begin[k + 1]) ++k;
-            const int c = n - g.col_begin[k];
-            const int h = c / g.hd, d = c - h * g.hd;
-            const float bv = HAS_BIAS ? g.bias[n] : 0.f;
-            const bool has_sb = g.sbias[k] != nullptr;
-            const float sb = has_sb ? g.sbias[k][c] : 0.f;
-            const bool fr = (g.frag >> k) & 1;
-            float* __restrict__ col = g.dst[k] + ((long long)h * g.S) * g.hd + (fr ? lbr_frag_offset(0, d, g.hd) : d);
-            const long long bstride = (long long)g.Hs[k] * g.S * g.hd;
-#pragma unroll
-            for (int i = 0; i < FM; ++i) {
-                const int mb = mw + i * 16 + rq;
-                const int b0 = mb / g.S, s0 = mb - b0 * g.S;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    if (mb + r >= M) continue;
-                    int b = b0, s = s0 + r;
-                    while (s >= g.S) {   // r < 4: at most one step unless S < 4
-                        s -= g.S;
-                        ++b;
-                    }
-                    float v = HAS_BIAS ? (acc[i][j][r] + bv) : g.alpha * acc[i][j][r];
-                    if (has_sb) v = v + sb;
-                    col[b * bstride + (fr ? lbr_frag_offset(s, 0, g.hd) : (long long)s * g.hd)] = v;
-                }
-            }
-        }
-        return;
-    }
-    if (FN % 2 == 0 && g.gF) {   // tiles with an odd block count never take a gated pair
-        // gated pair: blocks j (gate) and j+1 (up) of this wave hold the same 16
-        // output columns; out = act(gate (+ gated bias))·up, rounded like the
-        // unfused GEMM → SLICE → GATED_ACT chain
-        const int F = g.gF;
-        float* __restrict__ C = g.C + bz * (long long)M * F;
-#pragma unroll
-        for (int j = 0; j + 1 < FN; j += 2) {
-            const int o = tn * (TN / 2) + ((wn * FN + j) >> 1) * 16 + cl;
-            if (o >= F) continue;
-            const float bg = HAS_BIAS ? g.bias[g.gbase + o] : 0.f;
-            const float bu = HAS_BIAS ? g.bias[(g.gbase ? 0 : F) + o] : 0.f;
-            const float gb = g.gbias ? g.gbias[o] : 0.f;
-#pragma unroll
-            for (int i = 0; i < FM; ++i)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int m = mw + i * 16 + rq + r;
-                    if (m >= M) continue;
-                    float x = HAS_BIAS ? (acc[i][j][r] + bg) : g.alpha * acc[i][j][r];
-                    const float u = HAS_BIAS ? (acc[i][j + 1][r] + bu) : g.alpha * acc[i][j + 1][r];
-                    if (g.gbias) x = x + gb;
-                    const float a = g.gact == 0 ? lbr_silu(x) : lbr_gelu_tanh(x);
-                    C[(long long)m * F + o] = a * u;
-                }
-        }
-        return;
-    }
-    float* __restrict__ C = g.C + bz * g.sC;
-    const float* __restrict__ R = g.resid ? g.resid + bz * g.sC : nullptr;
-#pragma unroll
-    for (int j = 0; j < FN; ++j) {
-        const int n = nw + j * 16 + cl;
-        if (n >= N) continue;
-        const float bv = HAS_BIAS ? g.bias[n] : 0.f;
-#pragma unroll
-        for (int i = 0; i < FM; ++i) {
-            float rv[4] = {0.f, 0.f, 0.f, 0.f};
-            if (R) {
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int m = mw + i * 16 + rq + r;
-                    if (m < M) rv[r] = R[(long long)m * N + n];
-                }
-            }
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int m = mw + i * 16 + rq + r;
-                if (m >= M) continue;
-                float v = HAS_BIAS ? (acc[i][j][r] + bv) : g.alpha * acc[i][j][r];
-                if (R) v = v + rv[r];
-                C[(long long)m * N + n] = lbr_act(g.act, v);   // a fused activation never comes with resid
-            }
-        }
-    }
+    gemm_epilogue<TM, TN, WGM, WGN, 16, HAS_BIAS, !AHEADS && NORM == 0, NS * STAGE>(g, lds, acc, m0, n0, tn, wave,
+                                                                                    lane, bz, ks);
 }
 
 // ---------------------------------------------------------------- GEMV
@@ -938,89 +757,6 @@ __global__ __launch_bounds__(256) void gemv_n(GemmArgs g) {
     for (int k = 0; k < g.K; ++k) acc += a[k] * b[(long long)k * g.N + n];
     float* c = g.C + bz * g.sC;
     c[n] = HAS_BIAS ? acc + g.bias[n] : g.alpha * acc;
-}
-
-// Step::i: [0]=M [1]=N [2]=K [3]=batches [4]=trans_b [5]=fragment-major head splits [6]=has_bias
-//          [7]=sA [8]=sB [9]=sC [10]=ksplit [11]=kchunk [12]=float4 reduce
-//          [13]=1 (takes fused epilogues) [14]=DMA tile + 1 (0: gemm_mfma_f32)
-//          [19..30] head scatter, [31] activation, [32..34] gated pair, [35..37] A in
-//          head layout (see below) ; f[0] = alpha
-GemmArgs make_args(const Step& s) {
-    GemmArgs g;
-    g.A = (const float*)s.in[0];
-    g.B = (const float*)s.in[1];
-    g.bias = (const float*)s.in[2];
-    g.C = (float*)s.out;
-    g.M = (int)s.i[0];
-    g.N = (int)s.i[1];
-    g.K = (int)s.i[2];
-    g.sA = s.i[7];
-    g.sB = s.i[8];
-    g.sC = s.i[9];
-    g.alpha = s.f[0];
-    g.tiles_m = (g.M + BM - 1) / BM;
-    g.tiles_n = (g.N + BN - 1) / BN;
-    g.ksplit = s.i[10] > 1 ? (int)s.i[10] : 1;
-    g.kchunk = g.ksplit > 1 ? (int)s.i[11] : g.K;
-    g.W = (float*)s.ws;
-    // fused epilogue: in[3] = resid (gated pair: the GATED_ACT bias);
-    // i[19] = n_split, i[20..24] = col_begin, in[4..7] = dst, in[8..11] =
-    // split biases, i[25..28] = heads per split, i[29] = hd, i[30] = S,
-    // i[5] = splits stored fragment-major (bit k, set by the plan);
-    // i[31] = act; i[32] = gated F, i[33] = gated act, i[34] = gate half's first column
-    g.gF = (int)s.i[32];
-    g.gact = (int)s.i[33];
-    g.gbase = (int)s.i[34];
-    g.resid = g.gF ? nullptr : (const float*)s.in[3];
-    g.gbias = g.gF ? (const float*)s.in[3] : nullptr;
-    g.n_split = (int)s.i[19];
-    for (int k = 0; k < 5; ++k) g.col_begin[k] = (int)s.i[20 + k];
-    for (int k = 0; k < 4; ++k) {
-        g.dst[k] = (float*)s.in[4 + k];
-        g.sbias[k] = (const float*)s.in[8 + k];
-        g.Hs[k] = (int)s.i[25 + k];
-    }
-    g.hd = (int)s.i[29];
-    g.S = (int)s.i[30];
-    g.frag = (int)s.i[5];
-    // i[18] = head prologue parts (0: none; see lbr_merge_gemm_head_prologue), i[20..23]
-    // = their first columns and heads, i[24] = flags, i[25..26] = RoPE row strides over
-    // b and s, i[30] = S; in[4..5] outputs, in[6..7] norm weights, in[8..9] cos / sin,
-    // in[10..11] biases; f[2..3] eps
-    g.hp_parts = (int)s.i[18];
-    g.hp_flags = (int)s.i[24];
-    g.hp_S = (int)s.i[30];
-    for (int p = 0; p < 2; ++p) {
-        g.hp_col[p] = (int)s.i[20 + p];
-        g.hp_H[p] = (int)s.i[22 + p];
-        g.hp_out[p] = (float*)s.in[4 + p];
-        g.hp_w[p] = (const float*)s.in[6 + p];
-        g.hp_b[p] = (const float*)s.in[10 + p];
-        g.hp_eps[p] = s.f[2 + p];
-    }
-    g.hp_cos = (const float*)s.in[8];
-    g.hp_sin = (const float*)s.in[9];
-    g.hp_tst[0] = s.i[25];
-    g.hp_tst[1] = s.i[26];
-    g.act = (int)s.i[31];
-    // i[35..37] = A in head layout [B, H, S, hd]: H, S, hd (0: row-major A)
-    g.aH = (int)s.i[35];
-    g.aS = (int)s.i[36];
-    g.ahd = (int)s.i[37];
-    // i[15] = norm prologue (LBR_NORM_*), i[38] / i[39] = its weight / bias, f[1] = eps
-    g.nw = (const float*)(uintptr_t)s.i[38];
-    g.nb = (const float*)(uintptr_t)s.i[39];
-    g.neps = s.f[1];
-    // i[16] = norm after the split-K reduce (LBR_NORM_*), i[17] = its form
-    // (16·(1 wave / 2 block per row) + float4 per lane, + 256 when the K split
-    // was made for the norm); in[4] output, in[5]
-    // weight, in[6] LayerNorm bias, f[2] eps (the head-split fields are unused
-    // then: i[19] = 0)
-    g.nt_out = s.i[16] ? (float*)s.in[4] : nullptr;
-    g.nt_w = s.i[16] ? (const float*)s.in[5] : nullptr;
-    g.nt_b = s.i[16] ? (const float*)s.in[6] : nullptr;
-    g.nt_eps = s.f[2];
-    return g;
 }
 
 // C[i] = alpha·Σ_ks W[ks][i] (MATMUL) or Σ_ks W[ks][i] + bias[i % N]
@@ -1176,10 +912,21 @@ void launch_splitk_reduce(const Step& s, const GemmArgs& g, hipStream_t st) {
         hipLaunchKernelGGL((splitk_reduce<HAS_BIAS, false>), dim3(blocks), dim3(256), 0, st, g, total);
 }
 
+}  // namespace
+
+void gemm_reduce_ksplit(const Step& s, const GemmArgs& g, hipStream_t st) {
+    if (s.i[6]) launch_splitk_reduce<true>(s, g, st);
+    else launch_splitk_reduce<false>(s, g, st);
+}
+
+namespace {
+
 template <bool TRANS_B, bool VEC, bool HAS_BIAS>
 void launch_gemm_t(const Step& s, hipStream_t st) {
-    GemmArgs g = make_args(s);
+    GemmArgs g = gemm_make_args(s);
     if (g.M <= 0 || g.N <= 0) return;
+    g.tiles_m = (g.M + BM - 1) / BM;
+    g.tiles_n = (g.N + BN - 1) / BN;
     dim3 grid(g.tiles_m * g.tiles_n, g.ksplit, (unsigned)s.i[3]);
     hipLaunchKernelGGL((gemm_mfma_f32<TRANS_B, VEC, HAS_BIAS>), grid, dim3(NT), 0, st, g);
     if (g.ksplit > 1) launch_splitk_reduce<HAS_BIAS>(s, g, st);
@@ -1188,7 +935,7 @@ void launch_gemm_t(const Step& s, hipStream_t st) {
 template <int TM, int TN, int WGM, int WGN, int OCC, bool HAS_BIAS, bool AHEADS, int NORM = 0, int NS = 2,
           int KB = DBK>
 void launch_gemm_dma(const Step& s, hipStream_t st) {
-    GemmArgs g = make_args(s);
+    GemmArgs g = gemm_make_args(s);
     if (g.M <= 0 || g.N <= 0) return;
     g.tiles_m = (g.M + TM - 1) / TM;
     // a gated pair's tile covers TN/2 output columns (TN/2 gate + TN/2 up columns of C)
@@ -1199,6 +946,20 @@ void launch_gemm_dma(const Step& s, hipStream_t st) {
     if (g.ksplit > 1) launch_splitk_reduce<HAS_BIAS>(s, g, st);
 }
 
+// LBR_GEMM_TILE without its family suffix ("b3": a split-bf16 tile), null when unset.
+bool forced_split() {
+    const char* f = getenv("LBR_GEMM_TILE");
+    const size_t n = f ? strlen(f) : 0;
+    return n > 2 && strcmp(f + n - 2, "b3") == 0;
+}
+const char* forced_tile_name() {
+    const char* f = getenv("LBR_GEMM_TILE");
+    if (!f || !forced_split()) return f;
+    static thread_local char name[32];
+    snprintf(name, sizeof(name), "%.*s", (int)std::min<size_t>(strlen(f) - 2, sizeof(name) - 1), f);
+    return name;
+}
+
 // Tile shapes of the DMA GEMM: (TM, TN), workgroups resident per CU (LDS
 // and registers), and measured steady-state fraction of the fp32 MFMA peak.
 struct DmaTile {
@@ -1207,7 +968,9 @@ struct DmaTile {
     const char* name;
     bool model;    // chosen by choose_dma's model; the others only by measurement
                    // (gemm_dma_tune_candidates) or by name (LBR_GEMM_TILE)
-    bool pairs;    // an even number of 16-column blocks per wavefront (gated pairs)
+    bool pairs;    // an even number of MFMA column blocks per wavefront (gated pairs)
+    int split = -1;   // >= 0: the split-bf16 kernel's tile number (gemm_split_launcher)
+    double lat = 0.;  // split-bf16 tiles: µs a 16-wide K step takes a workgroup alone on its CU
 };
 constexpr DmaTile kDmaTiles[] = {
     {256, 256, 1, 8, 32, 0.94, "256x256", true, true},   // 8 wavefronts (4×2), 128 KB LDS
@@ -1239,22 +1002,58 @@ constexpr DmaTile kDmaTiles[] = {
     // against 51.5), so halving the barriers per K is not what those GEMMs lack
     {32, 96, 2, 4, 64, 0.80, "32x96k64", false, false},     // 64 KB LDS
     {64, 64, 2, 4, 64, 0.90, "64x64k64", false, true},      // 64 KB LDS
+    // Split-bf16 tiles (gemm_split.hip): efficiency as a multiple of the fp32 peak with
+    // every CU busy (4096×12288×4096: 248, 225, 225, 223, 193, 193, 160 TFLOP/s).
+    {256, 256, 1, 8, 32, 1.58, "256x256", true, true, 0, 1.50},
+    {256, 128, 1, 8, 32, 1.43, "256x128", true, true, 1, 0.86},
+    {128, 256, 1, 8, 32, 1.43, "128x256", true, true, 2, 0.86},
+    {128, 128, 3, 4, 32, 1.42, "128x128", true, true, 3, 0.59},
+    {128, 64, 4, 4, 32, 1.23, "128x64", true, false, 4, 0.47},
+    {64, 128, 4, 4, 32, 1.23, "64x128", true, true, 5, 0.47},
+    {64, 64, 6, 4, 32, 1.02, "64x64", true, false, 6, 0.39},
 };
 constexpr int kNumDmaTiles = sizeof(kDmaTiles) / sizeof(kDmaTiles[0]);
 
-// Tile shape and number of K ranges for the DMA GEMM.  Time model: the
-// busiest CU runs ceil(items / CUs) workgroups of TM·TN·kchunk MACs each
-// at the tile's efficiency, in rounds of `occ` resident workgroups that
-// each pay ~3 µs of first-load latency and epilogue; a K split adds writing
-// and re-reading the partial sums at ~5 TB/s plus a reduction launch.  A CU
-// left with fewer than 8 resident wavefronts (one 4-wavefront workgroup)
-// runs its tile at 0.9 of the efficiency: measured on GPT-2's FFN2 (1024 ×
-// 768 × 3072, 192 tiles of 64×64), one workgroup per CU took 55.8 µs, and
-// four K ranges, three workgroups per CU, took 46.3 µs.
-// LBR_GEMM_TILE (a tile name) and LBR_GEMM_KSPLIT override the choice.
-void choose_dma(long long M, long long N, int K, long long batches, int cus, int* tile, int* ksplit, int* kchunk) {
+// Time of an M×N×K GEMM (batches of it) on tile d with K ranges of `chunk` (s of them).
+// fp32 tiles: the busiest CU runs ceil(items / CUs) workgroups of TM·TN·chunk MACs each
+// at the tile's efficiency, in rounds of `occ` resident workgroups that each pay ~3 µs of
+// first-load latency and epilogue.  A CU left with fewer than 8 resident wavefronts (one
+// 4-wavefront workgroup) runs its tile at 0.9 of the efficiency: measured on GPT-2's FFN2
+// (1024 × 768 × 3072, 192 tiles of 64×64), one workgroup per CU took 55.8 µs, and four K
+// ranges, three workgroups per CU, took 46.3 µs.
+// Split-bf16 tiles: each round takes the larger of its workgroups' MFMA time and the chain
+// of one workgroup's K steps (`lat` each).  The MFMA rate is the power limit's: it rises as
+// CUs idle (256×256 tiles of 1024×6144×2560 on 96 CUs: 247 µs against 347 µs a round of a
+// full chip, 256×128 on 192: 164 against 191).
+// A K split adds writing and re-reading the partial sums at ~5 TB/s plus a reduction launch.
+double dma_time(const DmaTile& d, long long M, long long N, long long batches, int chunk, int s, int cus) {
     const double peak_cu = 157.3e12 / 256.0;
-    const char* force_tile = getenv("LBR_GEMM_TILE");
+    const long long items = ((M + d.tm - 1) / d.tm) * ((N + d.tn - 1) / d.tn) * batches * s;
+    const long long per_cu = (items + cus - 1) / cus;
+    double t = 0.;
+    if (d.split >= 0) {
+        const double busy = (double)items / (double)(per_cu * cus);
+        const double one = 2.0 * d.tm * d.tn * chunk / (d.eff * peak_cu) * (0.56 + 0.44 * busy);
+        const double chain = (double)((chunk + 15) / 16) * d.lat * 1e-6;
+        for (long long left = per_cu; left > 0; left -= d.occ)
+            t += std::max(chain, one * (double)std::min<long long>(left, d.occ)) + 3e-6;
+    } else {
+        const double eff = std::min<long long>(per_cu, d.occ) * d.waves < 8 ? 0.9 * d.eff : d.eff;
+        t = (double)per_cu * 2.0 * d.tm * d.tn * chunk / (eff * peak_cu);
+        t += (double)((per_cu + d.occ - 1) / d.occ) * 3e-6;   // per round: first DMA, epilogue
+    }
+    if (s > 1) t += (2.0 * s + 1.0) * M * N * batches * 4.0 / 5e12 + 4e-6;
+    return t;
+}
+
+// Whether a tile belongs to the split-bf16 family.
+bool is_split(int t) { return kDmaTiles[t].split >= 0; }
+
+// Tile shape and number of K ranges of the fp32 or the split-bf16 family by dma_time.
+// LBR_GEMM_TILE (a tile name) and LBR_GEMM_KSPLIT override the choice.  Returns its time.
+double choose_dma(bool split, long long M, long long N, int K, long long batches, int cus, int* tile, int* ksplit,
+                  int* kchunk) {
+    const char* force_tile = forced_tile_name();
     const char* force_ks = getenv("LBR_GEMM_KSPLIT");
     double best = 1e30;
     *tile = 1;
@@ -1263,9 +1062,9 @@ void choose_dma(long long M, long long N, int K, long long batches, int cus, int
     if (cus <= 0) cus = 256;
     for (int t = 0; t < kNumDmaTiles; ++t) {
         const DmaTile& d = kDmaTiles[t];
+        if (is_split(t) != split) continue;
         if (force_tile ? strcmp(force_tile, d.name) != 0 : !d.model) continue;
         if (K % d.kb) continue;
-        const long long tiles = ((M + d.tm - 1) / d.tm) * ((N + d.tn - 1) / d.tn) * batches;
         for (int s = 1; s <= 16; ++s) {
             const int chunk = ((K + s - 1) / s + d.kb - 1) / d.kb * d.kb;
             const int s_eff = (K + chunk - 1) / chunk;
@@ -1274,11 +1073,11 @@ void choose_dma(long long M, long long N, int K, long long batches, int cus, int
             } else if (s > 1 && (chunk < 256 || s_eff != s)) {
                 continue;
             }
-            const long long per_cu = (tiles * s_eff + cus - 1) / cus;
-            const double eff = std::min<long long>(per_cu, d.occ) * d.waves < 8 ? 0.9 * d.eff : d.eff;
-            double t_s = (double)per_cu * 2.0 * d.tm * d.tn * chunk / (eff * peak_cu);
-            t_s += (double)((per_cu + d.occ - 1) / d.occ) * 3e-6;   // per round: first DMA, epilogue
-            if (s_eff > 1) t_s += (2.0 * s_eff + 1.0) * M * N * batches * 4.0 / 5e12 + 4e-6;
+            // the split family's faster MFMAs favour more ranges than the fp32 one takes:
+            // never so many that lbr_execute_noalloc would refuse the node
+            if (split && !force_ks && s_eff > 1 && (double)s_eff * batches * M * N * 4.0 > (double)LBR_SCRATCH_BYTES)
+                continue;
+            double t_s = dma_time(d, M, N, batches, chunk, s_eff, cus);
             if (s_eff > 1 && !force_ks) t_s *= 1.05;   // split only for a clear gain
             if (t_s < best) {
                 best = t_s;
@@ -1288,10 +1087,26 @@ void choose_dma(long long M, long long N, int K, long long batches, int cus, int
             }
         }
     }
+    return best;
+}
+
+// Whether the GEMM takes the split-bf16 kernel: from 1.5e9 multiply-adds up, where both
+// kernels, each at its best tile and K ranges, were timed (µs a replayed node, fp32 / split):
+// 512×768×768 17.5 / 18.8, 512×3072×768 (1.2e9) 33.5 / 33.0, 256×2560×2560 (1.7e9) 41.6 /
+// 35.8, 1024×2304×768 47.7 / 39.0, 4096×1024×1024 76 / 62, 1024×2560×4096 195 / 120.
+// Below, a tile's few K steps are a chain of load, split and MFMA latencies on either
+// kernel, and the norm prologue and the one-kernel MLP (fp32) cover the smallest.
+// LBR_GEMM_SPLIT=0 keeps the fp32 kernel, =1 takes the split wherever its operands allow; a
+// tile forced by LBR_GEMM_TILE decides by its family ("b3" at its end: split).
+bool use_split(long long M, long long N, int K, long long batches) {
+    if (getenv("LBR_GEMM_TILE")) return forced_split();
+    if (const char* e = getenv("LBR_GEMM_SPLIT")) return atoi(e) != 0;
+    return (double)M * (double)N * (double)K * (double)batches > 1.5e9;
 }
 
 template <bool HAS_BIAS, bool AHEADS = false, int NORM = 0>
 step_fn dma_launcher(int tile) {
+    if (is_split(tile)) return NORM ? nullptr : gemm_split_launcher(kDmaTiles[tile].split, HAS_BIAS, AHEADS);
     switch (tile) {
         case 0:   // the norm prologue's registers do not fit beside the 256×256 accumulators
             if constexpr (NORM != 0) return nullptr;
@@ -1352,14 +1167,14 @@ int choose_ksplit(long long tiles, int K, long long MN, int cus, int* kchunk) {
 
 template <bool VEC, bool HAS_BIAS>
 void launch_gemv_t(const Step& s, hipStream_t st) {
-    GemmArgs g = make_args(s);
+    GemmArgs g = gemm_make_args(s);
     if (g.N <= 0) return;
     hipLaunchKernelGGL((gemv_t<VEC, HAS_BIAS>), dim3((g.N + 3) / 4, (unsigned)s.i[3]), dim3(256), 0, st, g);
 }
 
 template <bool HAS_BIAS>
 void launch_gemv_n(const Step& s, hipStream_t st) {
-    GemmArgs g = make_args(s);
+    GemmArgs g = gemm_make_args(s);
     if (g.N <= 0) return;
     hipLaunchKernelGGL((gemv_n<HAS_BIAS>), dim3((g.N + 255) / 256, (unsigned)s.i[3]), dim3(256), 0, st, g);
 }
@@ -1454,29 +1269,22 @@ bool gemm_dma_tile_pairs(int tile) {
     return tile >= 0 && tile < kNumDmaTiles && kDmaTiles[tile].pairs;
 }
 
-// The model's time for one K range on tile t (choose_dma's terms).
-static double dma_model_time(long long M, long long N, int K, int cus, int t) {
-    const DmaTile& d = kDmaTiles[t];
-    const double peak_cu = 157.3e12 / 256.0;
-    if (cus <= 0) cus = 256;
-    const long long tiles = ((M + d.tm - 1) / d.tm) * ((N + d.tn - 1) / d.tn);
-    const long long per_cu = (tiles + cus - 1) / cus;
-    const double eff = std::min<long long>(per_cu, d.occ) * d.waves < 8 ? 0.9 * d.eff : d.eff;
-    return (double)per_cu * 2.0 * d.tm * d.tn * K / (eff * peak_cu) + (double)((per_cu + d.occ - 1) / d.occ) * 3e-6;
-}
-
 int gemm_dma_tune_candidates(const Step& s, int* tiles, int cap) {
     int n = 0;
     if (!s.i[14] || s.i[10] > 1 || s.i[3] != 1) return 0;   // one batch, no K split
     // tiles the model prices at more than twice its best are not timed (the
     // 256×256 tile on a 1024-row GEMM, say): only near-ties need measuring
-    auto usable = [&](int t) { return dma_family_launcher(s, t) && s.i[2] % kDmaTiles[t].kb == 0; };
+    // (and only tiles of the step's own family: the two sum K in different orders)
+    auto usable = [&](int t) {
+        return is_split(t) == is_split((int)s.i[14] - 1) && dma_family_launcher(s, t) && s.i[2] % kDmaTiles[t].kb == 0;
+    };
+    const int cus = lbr_device_cus() > 0 ? lbr_device_cus() : 256;
+    auto time = [&](int t) { return dma_time(kDmaTiles[t], s.i[0], s.i[1], 1, (int)s.i[2], 1, cus); };
     double best = 1e30;
     for (int t = 0; t < kNumDmaTiles; ++t)
-        if (usable(t)) best = std::min(best, dma_model_time(s.i[0], s.i[1], (int)s.i[2], lbr_device_cus(), t));
+        if (usable(t)) best = std::min(best, time(t));
     for (int t = 0; t < kNumDmaTiles && n < cap; ++t)
-        if (usable(t) && dma_model_time(s.i[0], s.i[1], (int)s.i[2], lbr_device_cus(), t) <= 2.0 * best)
-            tiles[n++] = t;
+        if (usable(t) && time(t) <= 2.0 * best) tiles[n++] = t;
     return n;
 }
 
@@ -1484,9 +1292,10 @@ extern "C" const char* lbr_gemm_tile_name(int tile) {
     return tile >= 0 && tile < kNumDmaTiles ? kDmaTiles[tile].name : "";
 }
 
-int gemm_dma_tile_by_name(const char* name) {
+int gemm_dma_tile_by_name(const Step& s, const char* name) {
     for (int t = 0; t < kNumDmaTiles; ++t)
-        if (name && strcmp(name, kDmaTiles[t].name) == 0) return t;
+        if (name && s.i[14] && is_split(t) == is_split((int)s.i[14] - 1) && strcmp(name, kDmaTiles[t].name) == 0)
+            return t;
     return -1;
 }
 
@@ -1606,7 +1415,8 @@ int decode_matmul(const OpNode* n, Step* s) {
     const bool legacy = force_tile && strcmp(force_tile, "legacy") == 0;
     if (!legacy && trans_b && vec && K % DBK == 0 && M * K * 4 < (1LL << 31) && (long long)N * K * 4 < (1LL << 31)) {
         int tile = 1, ks = 1, kchunk = K;
-        choose_dma(M, N, K, batches, lbr_device_cus(), &tile, &ks, &kchunk);
+        const bool split = use_split(M, N, K, batches);
+        choose_dma(split, M, N, K, batches, lbr_device_cus(), &tile, &ks, &kchunk);
         s->i[10] = ks;
         s->i[11] = kchunk;
         s->i[14] = tile + 1;

@@ -336,6 +336,9 @@ struct Step {
     void* ws;                 // workspace assigned by the plan (shared by all steps)
 };
 
+// Workspace lbr_execute_noalloc has for a node (executor.hip).
+#define LBR_SCRATCH_BYTES ((size_t)48 << 20)
+
 // Number of compute units of the initialised device (0 before lbr_init).
 int lbr_device_cus();
 
@@ -418,8 +421,9 @@ bool gemm_dma_tile_pairs(int tile);
 bool gemm_dma_split2(Step* s);
 bool gemm_dma_retile(Step* s, int tile);
 bool gemm_dma_set_ksplit(Step* s, int ks);
-// Index of the DMA tile called `name` ("32x48", "64x64" ...), or -1.
-int gemm_dma_tile_by_name(const char* name);
+// Index of the DMA tile called `name` ("32x48", "64x64" ...) in the step's family (fp32 or
+// split-bf16), or -1.
+int gemm_dma_tile_by_name(const Step& s, const char* name);
 int gemm_dma_written(const Step& s, void** ptr, size_t* bytes, int cap);
 int decode_attention(const OpNode* n, Step* s);
 // Whether a decoded attention step can defer its store (its rows staged, then

@@ -1,0 +1,89 @@
+"""The split-bf16 GEMM (gemm_split.hip): every tile at its edges against a float64 closed form, its
+epilogues, and the results it hands to the fp32 matrix cores (infinities, NaN, tiny operands).
+
+The tolerance is the fp32 kernel's own: a dot product of K terms summed in fp32 is off by at most
+about K·2⁻²⁴ of Σ|a·b|; for the N(0,1) operands here that is below 1e-5 of the largest result."""
+
+import numpy as np
+import pytest
+
+import test_gpu_fused_epilogues as epilogues
+from conftest import normwise_rel
+from helpers import one_node_graph, randn, rng, run_gpu
+from runtime.ir import OpType
+from test_gpu_ops import _gemm_case
+
+pytestmark = pytest.mark.gpu
+
+TILES = ["256x256", "256x128", "128x256", "128x128", "128x64", "64x128", "64x64"]
+
+
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("M,N,K,batches", [(300, 520, 96, 1), (513, 257, 64, 1), (2, 3, 32, 1), (257, 130, 160, 3)])
+@pytest.mark.parametrize("with_bias", [False, True])
+def test_split_tiles(monkeypatch, tile, M, N, K, batches, with_bias):
+    monkeypatch.setenv("LBR_GEMM_TILE", tile + "b3")
+    monkeypatch.setenv("LBR_GEMM_KSPLIT", "1")
+    assert _gemm_case(M, N, K, True, batches, batches == 1, with_bias) == "gemm_dma_f32_nt"
+
+
+@pytest.mark.parametrize("tile,ks,M,N,K", [("256x256", 3, 200, 300, 960), ("64x64", 2, 70, 130, 64)])
+def test_split_ksplit(monkeypatch, tile, ks, M, N, K):
+    monkeypatch.setenv("LBR_GEMM_TILE", tile + "b3")
+    monkeypatch.setenv("LBR_GEMM_KSPLIT", str(ks))
+    _gemm_case(M, N, K, True, 1, True, True)
+
+
+@pytest.mark.parametrize("tile", ["256x256", "128x128", "64x128"])
+def test_split_epilogues(monkeypatch, tile):
+    epilogues.test_gemm_activation_epilogue(monkeypatch, OpType.GELU, True, tile + "b3", "1", 300, 520, 96)
+    epilogues.test_gemm_gated_epilogue(monkeypatch, tile + "b3", "silu", True, 0, True)
+    epilogues.test_transpose_gemm(monkeypatch, tile + "b3", "1", 12, 70, 8, 100, False, True)
+    epilogues.test_transpose_gemm(monkeypatch, tile + "b3", "1", 4, 300, 64, 200, True, True)
+
+
+def _run(a, b):
+    M, K = a.shape
+    g = one_node_graph(OpType.MATMUL, {"a": a[None]}, (1, M, b.shape[0]), {"transpose_b": True}, {"b": b})
+    return run_gpu(g, {"a": a[None]})[0]
+
+
+@pytest.mark.parametrize("tile", ["256x256", "64x64"])
+def test_split_is_exact_where_fp32_is(monkeypatch, tile):
+    """One term a row: the three planes add up to the fp32 value, to the last bit."""
+    monkeypatch.setenv("LBR_GEMM_TILE", tile + "b3")
+    monkeypatch.setenv("LBR_GEMM_KSPLIT", "1")
+    b = randn(rng(5), 130, 96) * np.exp2(rng(6).integers(-20, 20, (130, 96))).astype(np.float32)
+    np.testing.assert_array_equal(_run(np.eye(96, dtype=np.float32), b), b.T)
+
+
+@pytest.mark.parametrize("tile", ["256x256", "64x64"])
+def test_split_outside_range(monkeypatch, tile):
+    """Infinities, NaN, the largest finite values (infinite as bf16) and tiny operands (whose
+    low planes are no normal bf16 values) give what the fp32 kernel gives."""
+    monkeypatch.setenv("LBR_GEMM_KSPLIT", "1")
+    r = rng(11)
+    a, b = randn(r, 200, 96), randn(r, 150, 96)
+    a[3, 7] = np.inf
+    a[4, 9] = -np.inf
+    a[5, [1, 2]] = [np.inf, -np.inf]
+    a[70, 5] = np.nan
+    b[9, 40] = np.inf
+    b[9, :40] = 1.0
+    a[100] = 0.0
+    a[100, 11] = np.finfo(np.float32).max
+    b[:, 11] = np.sign(b[:, 11]) * 0.5
+    a[101] *= np.float32(1e-33)
+    a[102] *= np.float32(1e-36)
+    outs = {}
+    for t in (tile, tile + "b3"):
+        monkeypatch.setenv("LBR_GEMM_TILE", t)
+        outs[t] = _run(a, b)
+    x, y = outs[tile + "b3"], outs[tile]
+    np.testing.assert_array_equal(np.isnan(x), np.isnan(y))
+    np.testing.assert_array_equal(x[np.isinf(y)], y[np.isinf(y)])
+    np.testing.assert_array_equal(np.isinf(x), np.isinf(y))
+    ref = a.astype(np.float64) @ b.T.astype(np.float64)
+    for rows in ([100], [101], [102], [0, 1, 2, 60, 199]):   # each range by its own size
+        ok = np.isfinite(y[rows])
+        assert normwise_rel(x[rows][ok], ref[rows][ok]) <= 1e-5
