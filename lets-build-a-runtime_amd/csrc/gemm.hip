@@ -11,7 +11,7 @@
 // Three kernels: gemm_dma_f32 (below the register-staged one) takes trans_b GEMMs with K
 // a multiple of 32 — all the Linear layers of the workloads — with
 // v_mfma_f32_16x16x4_f32, direct-to-LDS loads and a tile shape chosen per GEMM; of those,
-// gemm_split_f32 (gemm_split.hip) takes the large ones (use_split) on the bf16 matrix
+// gemm_split_f32 (gemm_split.hip) takes the large ones (gemm_family) on the bf16 matrix
 // cores; gemm_mfma_f32 (v_mfma_f32_32x32x2_f32) takes the rest (B stored [K, N], ragged
 // K, unaligned operands).
 //
@@ -31,9 +31,9 @@
 // reuse the same A and B panels) hit the same L2.
 #include "gemm_common.h"
 
-#include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <string>
 
 // Step::i: [0]=M [1]=N [2]=K [3]=batches [4]=trans_b [5]=fragment-major head splits [6]=has_bias
 //          [7]=sA [8]=sB [9]=sC [10]=ksplit [11]=kchunk [12]=float4 reduce
@@ -946,18 +946,19 @@ void launch_gemm_dma(const Step& s, hipStream_t st) {
     if (g.ksplit > 1) launch_splitk_reduce<HAS_BIAS>(s, g, st);
 }
 
-// LBR_GEMM_TILE without its family suffix ("b3": a split-bf16 tile), null when unset.
-bool forced_split() {
+// Tile families: a tile's sums depend on its family alone (the order of the K terms), never
+// on its shape.
+enum Family { FP32, SPLIT };
+
+// LBR_GEMM_TILE: a tile name, with "b3" after it for the split-bf16 kernel.  *name gets the
+// tile name (empty when unset).
+Family forced_tile(std::string* name) {
     const char* f = getenv("LBR_GEMM_TILE");
-    const size_t n = f ? strlen(f) : 0;
-    return n > 2 && strcmp(f + n - 2, "b3") == 0;
-}
-const char* forced_tile_name() {
-    const char* f = getenv("LBR_GEMM_TILE");
-    if (!f || !forced_split()) return f;
-    static thread_local char name[32];
-    snprintf(name, sizeof(name), "%.*s", (int)std::min<size_t>(strlen(f) - 2, sizeof(name) - 1), f);
-    return name;
+    *name = f ? f : "";
+    const size_t n = name->size();
+    if (n <= 2 || name->compare(n - 2, 2, "b3") != 0) return FP32;
+    name->resize(n - 2);
+    return SPLIT;
 }
 
 // Tile shapes of the DMA GEMM: (TM, TN), workgroups resident per CU (LDS
@@ -969,8 +970,9 @@ struct DmaTile {
     bool model;    // chosen by choose_dma's model; the others only by measurement
                    // (gemm_dma_tune_candidates) or by name (LBR_GEMM_TILE)
     bool pairs;    // an even number of MFMA column blocks per wavefront (gated pairs)
-    int split = -1;   // >= 0: the split-bf16 kernel's tile number (gemm_split_launcher)
-    double lat = 0.;  // split-bf16 tiles: µs a 16-wide K step takes a workgroup alone on its CU
+    Family family = FP32;
+    int shape = 0;    // SPLIT: the tile's number (gemm_split_launcher)
+    double lat = 0.;  // SPLIT: µs a 16-wide K step takes a workgroup alone on its CU
 };
 constexpr DmaTile kDmaTiles[] = {
     {256, 256, 1, 8, 32, 0.94, "256x256", true, true},   // 8 wavefronts (4×2), 128 KB LDS
@@ -1004,13 +1006,13 @@ constexpr DmaTile kDmaTiles[] = {
     {64, 64, 2, 4, 64, 0.90, "64x64k64", false, true},      // 64 KB LDS
     // Split-bf16 tiles (gemm_split.hip): efficiency as a multiple of the fp32 peak with
     // every CU busy (4096×12288×4096: 248, 225, 225, 223, 193, 193, 160 TFLOP/s).
-    {256, 256, 1, 8, 32, 1.58, "256x256", true, true, 0, 1.50},
-    {256, 128, 1, 8, 32, 1.43, "256x128", true, true, 1, 0.86},
-    {128, 256, 1, 8, 32, 1.43, "128x256", true, true, 2, 0.86},
-    {128, 128, 3, 4, 32, 1.42, "128x128", true, true, 3, 0.59},
-    {128, 64, 4, 4, 32, 1.23, "128x64", true, false, 4, 0.47},
-    {64, 128, 4, 4, 32, 1.23, "64x128", true, true, 5, 0.47},
-    {64, 64, 6, 4, 32, 1.02, "64x64", true, false, 6, 0.39},
+    {256, 256, 1, 8, 32, 1.58, "256x256", true, true, SPLIT, 0, 1.50},
+    {256, 128, 1, 8, 32, 1.43, "256x128", true, true, SPLIT, 1, 0.86},
+    {128, 256, 1, 8, 32, 1.43, "128x256", true, true, SPLIT, 2, 0.86},
+    {128, 128, 3, 4, 32, 1.42, "128x128", true, true, SPLIT, 3, 0.59},
+    {128, 64, 4, 4, 32, 1.23, "128x64", true, false, SPLIT, 4, 0.47},
+    {64, 128, 4, 4, 32, 1.23, "64x128", true, true, SPLIT, 5, 0.47},
+    {64, 64, 6, 4, 32, 1.02, "64x64", true, false, SPLIT, 6, 0.39},
 };
 constexpr int kNumDmaTiles = sizeof(kDmaTiles) / sizeof(kDmaTiles[0]);
 
@@ -1031,7 +1033,7 @@ double dma_time(const DmaTile& d, long long M, long long N, long long batches, i
     const long long items = ((M + d.tm - 1) / d.tm) * ((N + d.tn - 1) / d.tn) * batches * s;
     const long long per_cu = (items + cus - 1) / cus;
     double t = 0.;
-    if (d.split >= 0) {
+    if (d.family != FP32) {
         const double busy = (double)items / (double)(per_cu * cus);
         const double one = 2.0 * d.tm * d.tn * chunk / (d.eff * peak_cu) * (0.56 + 0.44 * busy);
         const double chain = (double)((chunk + 15) / 16) * d.lat * 1e-6;
@@ -1046,14 +1048,12 @@ double dma_time(const DmaTile& d, long long M, long long N, long long batches, i
     return t;
 }
 
-// Whether a tile belongs to the split-bf16 family.
-bool is_split(int t) { return kDmaTiles[t].split >= 0; }
-
-// Tile shape and number of K ranges of the fp32 or the split-bf16 family by dma_time.
+// Tile shape and number of K ranges of one family by dma_time.
 // LBR_GEMM_TILE (a tile name) and LBR_GEMM_KSPLIT override the choice.  Returns its time.
-double choose_dma(bool split, long long M, long long N, int K, long long batches, int cus, int* tile, int* ksplit,
+double choose_dma(Family family, long long M, long long N, int K, long long batches, int cus, int* tile, int* ksplit,
                   int* kchunk) {
-    const char* force_tile = forced_tile_name();
+    std::string force_tile;
+    forced_tile(&force_tile);
     const char* force_ks = getenv("LBR_GEMM_KSPLIT");
     double best = 1e30;
     *tile = 1;
@@ -1062,9 +1062,9 @@ double choose_dma(bool split, long long M, long long N, int K, long long batches
     if (cus <= 0) cus = 256;
     for (int t = 0; t < kNumDmaTiles; ++t) {
         const DmaTile& d = kDmaTiles[t];
-        if (is_split(t) != split) continue;
-        if (force_tile ? strcmp(force_tile, d.name) != 0 : !d.model) continue;
-        if (K % d.kb) continue;
+        if (d.family != family) continue;
+        if (force_tile.empty() ? !d.model : force_tile != d.name) continue;
+        if (family == FP32 && K % d.kb) continue;   // the split kernel takes any K (RAGGED)
         for (int s = 1; s <= 16; ++s) {
             const int chunk = ((K + s - 1) / s + d.kb - 1) / d.kb * d.kb;
             const int s_eff = (K + chunk - 1) / chunk;
@@ -1075,7 +1075,7 @@ double choose_dma(bool split, long long M, long long N, int K, long long batches
             }
             // the split family's faster MFMAs favour more ranges than the fp32 one takes:
             // never so many that lbr_execute_noalloc would refuse the node
-            if (split && !force_ks && s_eff > 1 && (double)s_eff * batches * M * N * 4.0 > (double)LBR_SCRATCH_BYTES)
+            if (family != FP32 && !force_ks && s_eff > 1 && (double)s_eff * batches * M * N * 4.0 > (double)LBR_SCRATCH_BYTES)
                 continue;
             double t_s = dma_time(d, M, N, batches, chunk, s_eff, cus);
             if (s_eff > 1 && !force_ks) t_s *= 1.05;   // split only for a clear gain
@@ -1090,7 +1090,7 @@ double choose_dma(bool split, long long M, long long N, int K, long long batches
     return best;
 }
 
-// Whether the GEMM takes the split-bf16 kernel: from 1.5e9 multiply-adds up, where both
+// The family of a GEMM: the split-bf16 kernel from 1.5e9 multiply-adds up, where both
 // kernels, each at its best tile and K ranges, were timed (µs a replayed node, fp32 / split):
 // 512×768×768 17.5 / 18.8, 512×3072×768 (1.2e9) 33.5 / 33.0, 256×2560×2560 (1.7e9) 41.6 /
 // 35.8, 1024×2304×768 47.7 / 39.0, 4096×1024×1024 76 / 62, 1024×2560×4096 195 / 120.
@@ -1098,15 +1098,17 @@ double choose_dma(bool split, long long M, long long N, int K, long long batches
 // kernel, and the norm prologue and the one-kernel MLP (fp32) cover the smallest.
 // LBR_GEMM_SPLIT=0 keeps the fp32 kernel, =1 takes the split wherever its operands allow; a
 // tile forced by LBR_GEMM_TILE decides by its family ("b3" at its end: split).
-bool use_split(long long M, long long N, int K, long long batches) {
-    if (getenv("LBR_GEMM_TILE")) return forced_split();
-    if (const char* e = getenv("LBR_GEMM_SPLIT")) return atoi(e) != 0;
-    return (double)M * (double)N * (double)K * (double)batches > 1.5e9;
+Family gemm_family(long long M, long long N, int K, long long batches) {
+    std::string name;
+    if (getenv("LBR_GEMM_TILE")) return forced_tile(&name);
+    if (const char* e = getenv("LBR_GEMM_SPLIT")) return atoi(e) != 0 ? SPLIT : FP32;
+    return (double)M * (double)N * (double)K * (double)batches > 1.5e9 ? SPLIT : FP32;
 }
 
 template <bool HAS_BIAS, bool AHEADS = false, int NORM = 0>
 step_fn dma_launcher(int tile) {
-    if (is_split(tile)) return NORM ? nullptr : gemm_split_launcher(kDmaTiles[tile].split, HAS_BIAS, AHEADS);
+    if (kDmaTiles[tile].family != FP32)
+        return NORM ? nullptr : gemm_split_launcher(kDmaTiles[tile].shape, HAS_BIAS, AHEADS);
     switch (tile) {
         case 0:   // the norm prologue's registers do not fit beside the 256×256 accumulators
             if constexpr (NORM != 0) return nullptr;
@@ -1269,6 +1271,9 @@ bool gemm_dma_tile_pairs(int tile) {
     return tile >= 0 && tile < kNumDmaTiles && kDmaTiles[tile].pairs;
 }
 
+// Whether tile t sums K in the order of the step's own tile.
+static bool same_family(const Step& s, int t) { return kDmaTiles[t].family == kDmaTiles[s.i[14] - 1].family; }
+
 int gemm_dma_tune_candidates(const Step& s, int* tiles, int cap) {
     int n = 0;
     if (!s.i[14] || s.i[10] > 1 || s.i[3] != 1) return 0;   // one batch, no K split
@@ -1276,7 +1281,7 @@ int gemm_dma_tune_candidates(const Step& s, int* tiles, int cap) {
     // 256×256 tile on a 1024-row GEMM, say): only near-ties need measuring
     // (and only tiles of the step's own family: the two sum K in different orders)
     auto usable = [&](int t) {
-        return is_split(t) == is_split((int)s.i[14] - 1) && dma_family_launcher(s, t) && s.i[2] % kDmaTiles[t].kb == 0;
+        return same_family(s, t) && dma_family_launcher(s, t) && s.i[2] % kDmaTiles[t].kb == 0;
     };
     const int cus = lbr_device_cus() > 0 ? lbr_device_cus() : 256;
     auto time = [&](int t) { return dma_time(kDmaTiles[t], s.i[0], s.i[1], 1, (int)s.i[2], 1, cus); };
@@ -1294,8 +1299,7 @@ extern "C" const char* lbr_gemm_tile_name(int tile) {
 
 int gemm_dma_tile_by_name(const Step& s, const char* name) {
     for (int t = 0; t < kNumDmaTiles; ++t)
-        if (name && s.i[14] && is_split(t) == is_split((int)s.i[14] - 1) && strcmp(name, kDmaTiles[t].name) == 0)
-            return t;
+        if (name && s.i[14] && same_family(s, t) && strcmp(name, kDmaTiles[t].name) == 0) return t;
     return -1;
 }
 
@@ -1415,14 +1419,31 @@ int decode_matmul(const OpNode* n, Step* s) {
     const bool legacy = force_tile && strcmp(force_tile, "legacy") == 0;
     if (!legacy && trans_b && vec && K % DBK == 0 && M * K * 4 < (1LL << 31) && (long long)N * K * 4 < (1LL << 31)) {
         int tile = 1, ks = 1, kchunk = K;
-        const bool split = use_split(M, N, K, batches);
-        choose_dma(split, M, N, K, batches, lbr_device_cus(), &tile, &ks, &kchunk);
+        choose_dma(gemm_family(M, N, K, batches), M, N, K, batches, lbr_device_cus(), &tile, &ks, &kchunk);
         s->i[10] = ks;
         s->i[11] = kchunk;
         s->i[14] = tile + 1;
         s->ws_bytes = ks > 1 ? (size_t)ks * batches * M * N * sizeof(float) : 0;
         s->run = has_bias ? dma_launcher<true>(tile) : dma_launcher<false>(tile);
         s->name = "gemm_dma_f32_nt";
+        return LBR_OK;
+    }
+    // B [N, K] with K a multiple of 4 but not of 32, whole 16-byte rows: the split kernel
+    // with its columns past K read as zero, at any size; it has a tile for small grids where
+    // the register-staged kernel has 128×128 alone (µs, split against register-staged:
+    // 231×600×200 9.9 / 20.1, 231×200×712 11.3 / 55, 5×30×20 4.2 / 5.0, 3×1000×4100 15.6 / 30,
+    // 1000×4100×2564 145 / 260).  The step keeps the
+    // register-staged kernel's name and epilogues (residual, head scatter).
+    const bool ragged_split = trans_b && vec && M * K * 4 < (1LL << 31) && (long long)N * K * 4 < (1LL << 31) &&
+                              (force_tile || getenv("LBR_GEMM_SPLIT") ? gemm_family(M, N, K, batches) == SPLIT : true);
+    if (ragged_split) {
+        int tile = 0, ks = 1, kchunk = K;
+        choose_dma(SPLIT, M, N, K, batches, lbr_device_cus(), &tile, &ks, &kchunk);
+        s->i[10] = ks;
+        s->i[11] = kchunk;
+        s->ws_bytes = ks > 1 ? (size_t)ks * batches * M * N * sizeof(float) : 0;
+        s->run = has_bias ? dma_launcher<true>(tile) : dma_launcher<false>(tile);
+        s->name = "gemm_mfma_f32_nt";
         return LBR_OK;
     }
     {

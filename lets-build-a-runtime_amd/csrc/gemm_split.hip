@@ -284,8 +284,12 @@ void launch(const Step& s, hipStream_t st) {
     g.tiles_m = (g.M + TM - 1) / TM;
     g.tiles_n = g.gF ? (g.gF + TN / 2 - 1) / (TN / 2) : (g.N + TN - 1) / TN;
     const dim3 grid(g.tiles_m * g.tiles_n, g.ksplit, (unsigned)s.i[3]);
-    hipLaunchKernelGGL((gemm_split_f32<TM, TN, WGM, WGN, OCC, HAS_BIAS, AHEADS, false>), grid, dim3(64 * WGM * WGN), 0,
-                       st, g);
+    if (g.K % 16 == 0)
+        hipLaunchKernelGGL((gemm_split_f32<TM, TN, WGM, WGN, OCC, HAS_BIAS, AHEADS, false>), grid,
+                           dim3(64 * WGM * WGN), 0, st, g);
+    else if constexpr (!AHEADS)   // A in head layout: K is a multiple of 32
+        hipLaunchKernelGGL((gemm_split_f32<TM, TN, WGM, WGN, OCC, HAS_BIAS, false, true>), grid,
+                           dim3(64 * WGM * WGN), 0, st, g);
     if (g.ksplit > 1) gemm_reduce_ksplit(s, g, st);
 }
 
