@@ -128,12 +128,18 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, float* lds, con
                                               int wave, int lane, long long bz, int ks) {
     constexpr int NW = WGM * WGN;
     constexpr int RG = TM / WGM / (CB == 16 ? 16 : 8), CG = TN / WGN / CB;
-    const int M = g.M, N = g.N;
+    // the fields the loops use, read once (the stores below may alias what g refers to, so the
+    // compiler would read them again after each)
+    const int M = g.M, N = g.N, act = g.act, seq = g.S, hdim = g.hd, gact = g.gact;
+    const float alpha = g.alpha;
+    const float* __restrict__ bias = g.bias;
+    const float* __restrict__ gbias = g.gbias;
     const int wm = wave / WGN, wn = wave % WGN;
     const int cl = lane & (CB - 1);
-    const int mw = m0 + wm * (TM / WGM), nw = n0 + wn * (TN / WGN);
-    // first row of a lane's row group i, within the wavefront's block
-    auto row0 = [&](int i) { return CB == 16 ? i * 16 + (lane >> 4) * 4 : i * 8 + (lane >> 5) * 4; };
+    // a lane's row group i starts at row mw + i·RS
+    constexpr int RS = CB == 16 ? 16 : 8;
+    const int lr = CB == 16 ? (lane >> 4) * 4 : (lane >> 5) * 4;
+    const int mw = m0 + wm * (TM / WGM) + lr, nw = n0 + wn * (TN / WGN);
     if constexpr (HEADP && TM == 64 && TN == 128 && WGM == 2 && WGN == 2) {
         int p = -1;
         for (int q = 0; q < g.hp_parts; ++q)
@@ -148,13 +154,13 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, float* lds, con
 #pragma unroll
             for (int j = 0; j < CG; ++j) {
                 const int c = wn * (TN / WGN) + j * CB + cl;
-                const float bv = HAS_BIAS ? g.bias[n0 + c] : 0.f;
+                const float bv = HAS_BIAS ? bias[n0 + c] : 0.f;
 #pragma unroll
                 for (int i = 0; i < RG; ++i)
 #pragma unroll
                     for (int r = 0; r < 4; ++r)
-                        lds[(wm * (TM / WGM) + row0(i) + r) * TS + c] =
-                            HAS_BIAS ? (acc_at(acc, i, j, r) + bv) : g.alpha * acc_at(acc, i, j, r);
+                        lds[(wm * (TM / WGM) + i * RS + lr + r) * TS + c] =
+                            HAS_BIAS ? (acc_at(acc, i, j, r) + bv) : alpha * acc_at(acc, i, j, r);
             }
             __syncthreads();
             const int H = g.hp_H[p], h = (n0 - g.hp_col[p]) / TN, S = g.hp_S;
@@ -201,7 +207,7 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, float* lds, con
             for (int i = 0; i < RG; ++i)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const int m = mw + row0(i) + r;
+                    const int m = mw + i * RS + r;
                     if (m < M) Wp[(long long)m * N + n] = acc_at(acc, i, j, r);
                 }
         }
@@ -217,28 +223,28 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, float* lds, con
             int k = 0;
             while (k + 1 < g.n_split && n >= g.col_begin[k + 1]) ++k;
             const int c = n - g.col_begin[k];
-            const int h = c / g.hd, d = c - h * g.hd;
-            const float bv = HAS_BIAS ? g.bias[n] : 0.f;
+            const int h = c / hdim, d = c - h * hdim;
+            const float bv = HAS_BIAS ? bias[n] : 0.f;
             const bool has_sb = g.sbias[k] != nullptr;
             const float sb = has_sb ? g.sbias[k][c] : 0.f;
             const bool fr = (g.frag >> k) & 1;
-            float* __restrict__ col = g.dst[k] + ((long long)h * g.S) * g.hd + (fr ? lbr_frag_offset(0, d, g.hd) : d);
-            const long long bstride = (long long)g.Hs[k] * g.S * g.hd;
+            float* __restrict__ col = g.dst[k] + ((long long)h * seq) * hdim + (fr ? lbr_frag_offset(0, d, hdim) : d);
+            const long long bstride = (long long)g.Hs[k] * seq * hdim;
 #pragma unroll
             for (int i = 0; i < RG; ++i) {
-                const int mb = mw + row0(i);
-                const int b0 = mb / g.S, s0 = mb - b0 * g.S;
+                const int mb = mw + i * RS;
+                const int b0 = mb / seq, s0 = mb - b0 * seq;
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     if (mb + r >= M) continue;
                     int b = b0, s = s0 + r;
-                    while (s >= g.S) {   // r < 4: at most one step unless S < 4
-                        s -= g.S;
+                    while (s >= seq) {   // r < 4: at most one step unless S < 4
+                        s -= seq;
                         ++b;
                     }
-                    float v = HAS_BIAS ? (acc_at(acc, i, j, r) + bv) : g.alpha * acc_at(acc, i, j, r);
+                    float v = HAS_BIAS ? (acc_at(acc, i, j, r) + bv) : alpha * acc_at(acc, i, j, r);
                     if (has_sb) v = v + sb;
-                    col[b * bstride + (fr ? lbr_frag_offset(s, 0, g.hd) : (long long)s * g.hd)] = v;
+                    col[b * bstride + (fr ? lbr_frag_offset(s, 0, hdim) : (long long)s * hdim)] = v;
                 }
             }
         }
@@ -254,19 +260,19 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, float* lds, con
         for (int j = 0; j + 1 < CG; j += 2) {
             const int o = tn * (TN / 2) + ((wn * CG + j) >> 1) * CB + cl;
             if (o >= F) continue;
-            const float bg = HAS_BIAS ? g.bias[g.gbase + o] : 0.f;
-            const float bu = HAS_BIAS ? g.bias[(g.gbase ? 0 : F) + o] : 0.f;
-            const float gb = g.gbias ? g.gbias[o] : 0.f;
+            const float bg = HAS_BIAS ? bias[g.gbase + o] : 0.f;
+            const float bu = HAS_BIAS ? bias[(g.gbase ? 0 : F) + o] : 0.f;
+            const float gb = gbias ? gbias[o] : 0.f;
 #pragma unroll
             for (int i = 0; i < RG; ++i)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const int m = mw + row0(i) + r;
+                    const int m = mw + i * RS + r;
                     if (m >= M) continue;
-                    float x = HAS_BIAS ? (acc_at(acc, i, j, r) + bg) : g.alpha * acc_at(acc, i, j, r);
-                    const float u = HAS_BIAS ? (acc_at(acc, i, j + 1, r) + bu) : g.alpha * acc_at(acc, i, j + 1, r);
-                    if (g.gbias) x = x + gb;
-                    const float a = g.gact == 0 ? lbr_silu(x) : lbr_gelu_tanh(x);
+                    float x = HAS_BIAS ? (acc_at(acc, i, j, r) + bg) : alpha * acc_at(acc, i, j, r);
+                    const float u = HAS_BIAS ? (acc_at(acc, i, j + 1, r) + bu) : alpha * acc_at(acc, i, j + 1, r);
+                    if (gbias) x = x + gb;
+                    const float a = gact == 0 ? lbr_silu(x) : lbr_gelu_tanh(x);
                     C[(long long)m * F + o] = a * u;
                 }
         }
@@ -278,24 +284,21 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, float* lds, con
     for (int j = 0; j < CG; ++j) {
         const int n = nw + j * CB + cl;
         if (n >= N) continue;
-        const float bv = HAS_BIAS ? g.bias[n] : 0.f;
+        const float bv = HAS_BIAS ? bias[n] : 0.f;
 #pragma unroll
         for (int i = 0; i < RG; ++i) {
             float rv[4] = {0.f, 0.f, 0.f, 0.f};
-            if (R) {
+            if (R) {   // rows clamped, not skipped: the four loads go out together
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int m = mw + row0(i) + r;
-                    if (m < M) rv[r] = R[(long long)m * N + n];
-                }
+                for (int r = 0; r < 4; ++r) rv[r] = R[(long long)min(mw + i * RS + r, M - 1) * N + n];
             }
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int m = mw + row0(i) + r;
+                const int m = mw + i * RS + r;
                 if (m >= M) continue;
-                float v = HAS_BIAS ? (acc_at(acc, i, j, r) + bv) : g.alpha * acc_at(acc, i, j, r);
+                float v = HAS_BIAS ? (acc_at(acc, i, j, r) + bv) : alpha * acc_at(acc, i, j, r);
                 if (R) v = v + rv[r];
-                C[(long long)m * N + n] = lbr_act(g.act, v);   // a fused activation never comes with resid
+                C[(long long)m * N + n] = lbr_act(act, v);   // a fused activation never comes with resid
             }
         }
     }
