@@ -492,22 +492,35 @@ struct Rope {
     const void* out;
 };
 
-// The 7-node rotate_half RoPE window (HF apply_rotary_pos_emb as exported:
-// q·cos, q[..., :half], q[..., half:], −, cat, ·sin, +) on x = [B, H, S, hd].
+// The 7-node rotate_half RoPE window on x = [B, H, S, hd]: q·cos, q[..., :half],
+// q[..., half:], −, cat, ·sin, +, the sum last and the others in whatever order the
+// exported model has them (HF's apply_rotary_pos_emb takes both halves first; a model that
+// writes cat((−q[..., half:], q[..., :half])) negates between its slices).
 bool match_rope(const OpNode* nodes, int n, int q, const void* x, int B, int H, int S, int hd, Rope* r,
                 std::vector<Rng>* inter) {
     if (q + 7 > n || hd % 2) return false;
     const int half = hd / 2;
     const long long rows = (long long)B * H * S;
-    const OpNode* mc = &nodes[q];
-    const OpNode* s1 = &nodes[q + 1];
-    const OpNode* s2 = &nodes[q + 2];
-    const OpNode* ng = &nodes[q + 3];
-    const OpNode* ct = &nodes[q + 4];
-    const OpNode* ms = &nodes[q + 5];
+    const OpNode *mc = nullptr, *s1 = nullptr, *s2 = nullptr, *ng = nullptr, *ct = nullptr, *ms = nullptr;
+    const Rng xr = rng(x, rows * hd * 4);
+    bool x_over = false;   // a node of the window has written over x (the planner reuses it once dead)
+    for (int k = 0; k < 7; ++k) {
+        const OpNode* nd = &nodes[q + k];
+        if (!is_f32(nd) || nd->n_inputs < 1) return false;
+        if (k == 6) break;   // the sum
+        // the rotated half's product reads the CAT, which may lie where x was
+        const OpNode** role = nd->op == OP_MUL     ? (ct && nd->inputs[0] == ct->output ? &ms : &mc)
+                              : nd->op == OP_SLICE ? (nd->extra[2] == 0 ? &s1 : &s2)
+                              : nd->op == OP_NEG   ? &ng
+                              : nd->op == OP_CAT   ? &ct
+                                                   : nullptr;
+        if (!role || *role || (x_over && (role == &mc || role == &s1 || role == &s2)) || (role == &ng && !s2) ||
+            (role == &ct && !(s1 && ng)))
+            return false;
+        *role = nd;
+        x_over = x_over || overlap(out_rng(nd), xr);
+    }
     const OpNode* ad = &nodes[q + 6];
-    for (int k = 0; k < 7; ++k)
-        if (!is_f32(&nodes[q + k])) return false;
     const int shape[4] = {B, H, S, hd};
     auto bcast_mul = [&](const OpNode* m, const void* a, long long* st) {
         // SUB/MUL/DIV extras: [2 = broadcast, ndim, a strides, b strides, out shape]
