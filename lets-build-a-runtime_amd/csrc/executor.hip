@@ -394,7 +394,7 @@ static int relay_gated_outputs(lbr_plan* p) {
         const Step& s = p->steps[i];
         if (s.fuse_kind != LBR_FUSE_GEMM_GATED || s.i[28] != 1) continue;
         if (i + 1 >= p->steps.size() || p->steps[i + 1].in[0] != s.out || !p->steps[i + 1].name ||
-            strncmp(p->steps[i + 1].name, "gemm_", 5) != 0) {
+            (strncmp(p->steps[i + 1].name, "gemm_", 5) != 0 && strncmp(p->steps[i + 1].name, "gemv_", 5) != 0)) {
             lbr_set_error("lbr_plan_create: the gated GEMM at node %d is not followed by the GEMM reading its "
                           "output as A", s.node_index);
             return LBR_ERR_INVALID;

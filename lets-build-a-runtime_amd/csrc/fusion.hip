@@ -753,7 +753,14 @@ bool gemm_step(const OpNode* g, Step* st) {
         lbr_set_error("");
         return false;
     }
-    return st->i[13] == 1;
+    return st->i[13] == 1 || st->i[13] == 2;
+}
+
+// Whether a GEMM step's kernel applies an activation, or a gated pair, in its epilogue: the
+// DMA kernels (pairs: tiles with an even number of blocks, no K split) and the one-row GEMV.
+bool gemm_takes_act(const Step& s) { return s.i[14] || s.i[13] == 2; }
+bool gemm_takes_pairs(const Step& s) {
+    return s.i[3] == 1 && s.i[10] <= 1 && (s.i[13] == 2 || (s.i[14] && gemm_dma_tile_pairs((int)s.i[14] - 1)));
 }
 
 // TRANSPOSE_GEMM at node i: T = TRANSPOSE(O [B, H, S, hd] → [B, S, H, hd]) is the A
@@ -880,7 +887,7 @@ bool match_mlp(const OpNode* nodes, int n, int i, bool free, const std::vector<R
         !is_f32(g2) || node_total(ac) != node_total(g1) || g2->n_inputs < 2 || g2->inputs[0] != ac->output)
         return false;
     Step s1, s2;
-    if (!gemm_step(g1, &s1) || !gemm_step(g2, &s2)) return false;
+    if (!gemm_step(g1, &s1) || !gemm_step(g2, &s2) || s1.i[13] != 1 || s2.i[13] != 1) return false;
     const long long M = s1.i[0], D = s1.i[2], H = s1.i[1], D2 = s2.i[1];
     if (s1.i[3] != 1 || s2.i[3] != 1 || !s1.i[4] || !s2.i[4] || s2.i[0] != M || s2.i[2] != H) return false;
     if (!mlp_shape_ok(M, D, H, D2) || 2.0 * (double)M * (double)(H * D + D2 * H) > 33554432.0) return false;
@@ -1119,8 +1126,7 @@ int lbr_find_fusions(const OpNode* nodes, int n, const void* const* live_ptr, co
             }
             // GEMM_GATED: C [rows, 2F] → SLICE(C, last dim) × 2 → GATED_ACT(gate, [bias], up), one
             // slice the column half [0, F) and the other [F, 2F); DMA kernel, one batch, no K split
-            if (gs.i[14] && gemm_dma_tile_pairs((int)gs.i[14] - 1) && gs.i[3] == 1 && gs.i[10] <= 1 &&
-                gs.i[1] % 2 == 0 && i + 3 < n && is_f32(nd)) {
+            if (gemm_takes_pairs(gs) && gs.i[1] % 2 == 0 && i + 3 < n && is_f32(nd)) {
                 const long long rows = gs.i[0];
                 const int N = (int)gs.i[1], F = N / 2;
                 const OpNode* s1 = &nodes[i + 1];
@@ -1170,8 +1176,8 @@ int lbr_find_fusions(const OpNode* nodes, int n, const void* const* live_ptr, co
                     }
                 }
             }
-            // GEMM_ACT: C → RELU | GELU | SILU (DMA kernel)
-            if (gs.i[14] && i + 1 < n) {
+            // GEMM_ACT: C → RELU | GELU | SILU (DMA kernel, GEMV)
+            if (gemm_takes_act(gs) && i + 1 < n) {
                 const OpNode* ac = &nodes[i + 1];
                 const int act = ac->op == OP_RELU ? LBR_ACT_RELU
                               : ac->op == OP_GELU ? LBR_ACT_GELU
@@ -1494,8 +1500,7 @@ int lbr_fused_step(const OpNode* nodes, const FusedRun& f, Step* s) {
     } else if (f.kind == LBR_FUSE_GEMM_ACT || f.kind == LBR_FUSE_GEMM_GATED) {
         int rc = decode_matmul(&nodes[f.first + (f.norm ? 1 : 0)], s);
         if (rc) return rc;
-        if (!s->i[14] || (f.kind == LBR_FUSE_GEMM_GATED &&
-                          (s->i[10] > 1 || s->i[3] != 1 || !gemm_dma_tile_pairs((int)s->i[14] - 1)))) {
+        if (!gemm_takes_act(*s) || (f.kind == LBR_FUSE_GEMM_GATED && !gemm_takes_pairs(*s))) {
             lbr_set_error("fusion: GEMM node %d is not on the DMA path without a K split", f.first);
             return LBR_ERR_INVALID;
         }
@@ -1503,27 +1508,27 @@ int lbr_fused_step(const OpNode* nodes, const FusedRun& f, Step* s) {
         if (f.kind == LBR_FUSE_GEMM_ACT) {
             s->i[31] = f.act;
             s->i[12] = s->i[12] && lbr_aligned(f.out, 16);
-            s->name = "gemm_dma_f32_nt+act";
+            s->name = s->i[14] ? "gemm_dma_f32_nt+act" : "gemv_t+act";
         } else {
             s->i[32] = f.gF;
             s->i[33] = f.gact;
             s->i[34] = f.gate_base;
             s->in[3] = f.gbias;
             s->i[28] = f.relay_out ? 1 : 0;   // relay_gated_outputs moves the output
-            s->name = "gemm_dma_f32_nt+gated";
+            s->name = s->i[14] ? "gemm_dma_f32_nt+gated" : "gemv_t+gated";
         }
     } else if (f.kind == LBR_FUSE_GEMM_RESID || f.kind == LBR_FUSE_GEMM_HEADS) {
         int rc = decode_matmul(&nodes[f.first + (f.norm ? 1 : 0)], s);
         if (rc) return rc;
-        if (s->i[13] != 1) {
-            lbr_set_error("fusion: GEMM node %d is not on the MFMA path", f.first);
+        if (s->i[13] != 1 && s->i[13] != 2) {
+            lbr_set_error("fusion: GEMM node %d has no fused epilogues", f.first);
             return LBR_ERR_INVALID;
         }
         if (f.kind == LBR_FUSE_GEMM_RESID) {
             s->in[3] = f.resid;
             s->out = (void*)f.out;
             s->i[12] = s->i[12] && lbr_aligned(f.out, 16);
-            s->name = s->i[14] ? "gemm_dma_f32_nt+resid" : s->i[4] ? "gemm_mfma_f32_nt+resid" : "gemm_mfma_f32_nn+resid";
+            s->name = s->i[13] == 2 ? "gemv_t+resid" : s->i[14] ? "gemm_dma_f32_nt+resid" : s->i[4] ? "gemm_mfma_f32_nt+resid" : "gemm_mfma_f32_nn+resid";
         } else {
             if (f.n_split < 1 || f.n_split > 4) {
                 lbr_set_error("fusion: %d head splits", f.n_split);
@@ -1539,7 +1544,7 @@ int lbr_fused_step(const OpNode* nodes, const FusedRun& f, Step* s) {
             s->i[20 + f.n_split] = f.col_begin[f.n_split - 1] + f.width[f.n_split - 1];
             s->i[29] = f.hd;
             s->i[30] = f.S;
-            s->name = s->i[14] ? "gemm_dma_f32_nt+heads" : s->i[4] ? "gemm_mfma_f32_nt+heads" : "gemm_mfma_f32_nn+heads";
+            s->name = s->i[13] == 2 ? "gemv_t+heads" : s->i[14] ? "gemm_dma_f32_nt+heads" : s->i[4] ? "gemm_mfma_f32_nt+heads" : "gemm_mfma_f32_nn+heads";
         }
     } else {
         s->in[0] = f.src;
@@ -1881,7 +1886,7 @@ bool lbr_merge_reduce_norm(Step* g, const Step& n) {
     // reduce never reads A)
     const bool tin = g->fuse_kind == LBR_FUSE_TRANSPOSE_GEMM;
     if ((g->fuse_kind != LBR_FUSE_GEMM_RESID && !tin) || !g->in[3] || (g->i[10] <= 1 && !split2) || g->i[3] != 1 ||
-        !g->i[12] || g->i[19] || g->i[32] || g->i[31] || g->i[16] || g->i[18] || !n.name)
+        !g->i[12] || g->i[19] || g->i[32] || g->i[31] || g->i[16] || g->i[18] || g->i[13] != 1 || !n.name)
         return false;
     const bool rms = strcmp(n.name, "rmsnorm") == 0;
     if (!rms && strcmp(n.name, "layernorm") != 0) return false;

@@ -37,7 +37,7 @@
 
 // Step::i: [0]=M [1]=N [2]=K [3]=batches [4]=trans_b [5]=fragment-major head splits [6]=has_bias
 //          [7]=sA [8]=sB [9]=sC [10]=ksplit [11]=kchunk [12]=float4 reduce
-//          [13]=1 (takes fused epilogues) [14]=DMA tile + 1 (0: gemm_mfma_f32)
+//          [13]=1 (takes fused epilogues; 2: gemv_t, which does too) [14]=DMA tile + 1 (0: gemm_mfma_f32)
 //          [19..30] head scatter, [31] activation, [32..34] gated pair, [35..37] A in
 //          head layout (see below) ; f[0] = alpha
 GemmArgs gemm_make_args(const Step& s) {
@@ -717,31 +717,63 @@ __global__ __launch_bounds__(64 * WGM * WGN, OCC) void gemm_dma_f32(GemmArgs g) 
 
 // ---------------------------------------------------------------- GEMV
 // M == 1 (decode): the reference switches to sgemv here (executor.c:217).
-// trans_b: one wavefront per output column, lanes stride over K.
+// trans_b: one wavefront per output column, lanes stride over K; bound by reading B (9728 x
+// 2560 rows: 17.4 µs, 5.7 TB/s).  The one value a column gives goes through the GEMMs' fused
+// epilogues (epi_store, activation, gated pair: a wavefront then takes a gate row and its up
+// row), so that a layer on one token does not spend a kernel of 2 µs and a gap of 1.5 µs to the
+// next on each addition, slice and product (width 2560, 32 heads, gated 9728, in one graph:
+// 14 kernels and 121 µs → 9 and 112).
+template <bool VEC, int R>
+__device__ __forceinline__ void gemv_rows(const float* __restrict__ a, const float* const (&b)[R], int K, int lane,
+                                          float (&acc)[R]) {
+    const int steps = VEC ? K / 4 : K;
+#pragma unroll
+    for (int r = 0; r < R; ++r) acc[r] = 0.f;
+    for (int k = lane; k < steps; k += 64) {
+        if (VEC) {
+            const float4 x = reinterpret_cast<const float4*>(a)[k];
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const float4 y = reinterpret_cast<const float4*>(b[r])[k];
+                acc[r] += (x.x * y.x + x.y * y.y) + (x.z * y.z + x.w * y.w);
+            }
+        } else {
+            const float x = a[k];
+#pragma unroll
+            for (int r = 0; r < R; ++r) acc[r] += x * b[r][k];
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) acc[r] = wave_sum(acc[r]);
+}
+
 template <bool VEC, bool HAS_BIAS>
 __global__ __launch_bounds__(256) void gemv_t(GemmArgs g) {
     const int lane = threadIdx.x & 63;
     const int n = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (n >= g.N) return;
     const long long bz = blockIdx.y;
-    const float* __restrict__ a = g.A + bz * g.sA;
-    const float* __restrict__ b = g.B + bz * g.sB + (long long)n * g.K;
-    float acc = 0.f;
-    if (VEC) {
-        const int k4 = g.K / 4;
-        const float4* a4 = reinterpret_cast<const float4*>(a);
-        const float4* b4 = reinterpret_cast<const float4*>(b);
-        for (int k = lane; k < k4; k += 64) {
-            const float4 x = a4[k], y = b4[k];
-            acc += (x.x * y.x + x.y * y.y) + (x.z * y.z + x.w * y.w);
-        }
-    } else {
-        for (int k = lane; k < g.K; k += 64) acc += a[k] * b[k];
-    }
-    acc = wave_sum(acc);
+    const float* const row[1] = {g.B + bz * g.sB + (long long)n * g.K};
+    float acc[1];
+    gemv_rows<VEC, 1>(g.A + bz * g.sA, row, g.K, lane, acc);
+    if (lane == 0) epi_store(g, bz, 0, n, lbr_act(g.act, HAS_BIAS ? acc[0] + g.bias[n] : g.alpha * acc[0]));
+}
+
+// Gated pair: out[j] = act(gate[j] (+ gated bias))·up[j], rounded as the unfused nodes would.
+template <bool VEC, bool HAS_BIAS>
+__global__ __launch_bounds__(256) void gemv_t_gated(GemmArgs g) {
+    const int lane = threadIdx.x & 63;
+    const int o = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (o >= g.gF) return;
+    const int ng = g.gbase + o, nu = (g.gbase ? 0 : g.gF) + o;
+    const float* const rows[2] = {g.B + (long long)ng * g.K, g.B + (long long)nu * g.K};
+    float acc[2];
+    gemv_rows<VEC, 2>(g.A, rows, g.K, lane, acc);
     if (lane == 0) {
-        float* c = g.C + bz * g.sC;
-        c[n] = HAS_BIAS ? acc + g.bias[n] : g.alpha * acc;
+        float x = HAS_BIAS ? acc[0] + g.bias[ng] : g.alpha * acc[0];
+        const float u = HAS_BIAS ? acc[1] + g.bias[nu] : g.alpha * acc[1];
+        if (g.gbias) x = x + g.gbias[o];
+        g.C[o] = (g.gact == 0 ? lbr_silu(x) : lbr_gelu_tanh(x)) * u;
     }
 }
 
@@ -1171,6 +1203,10 @@ template <bool VEC, bool HAS_BIAS>
 void launch_gemv_t(const Step& s, hipStream_t st) {
     GemmArgs g = gemm_make_args(s);
     if (g.N <= 0) return;
+    if (g.gF) {
+        hipLaunchKernelGGL((gemv_t_gated<VEC, HAS_BIAS>), dim3((g.gF + 3) / 4), dim3(256), 0, st, g);
+        return;
+    }
     hipLaunchKernelGGL((gemv_t<VEC, HAS_BIAS>), dim3((g.N + 3) / 4, (unsigned)s.i[3]), dim3(256), 0, st, g);
 }
 
@@ -1403,6 +1439,7 @@ int decode_matmul(const OpNode* n, Step* s) {
             s->run = vec ? (has_bias ? launch_gemv_t<true, true> : launch_gemv_t<true, false>)
                          : (has_bias ? launch_gemv_t<false, true> : launch_gemv_t<false, false>);
             s->name = "gemv_t";
+            if (batches == 1) s->i[13] = 2;   // takes the fused epilogues too
         } else {
             s->run = has_bias ? launch_gemv_n<true> : launch_gemv_n<false>;
             s->name = "gemv_n";
