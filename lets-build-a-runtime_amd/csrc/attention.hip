@@ -1141,6 +1141,41 @@ void launch_attn(const Step& s, hipStream_t st) {
                        g);
 }
 
+// One token (S = 1, no mask): a wavefront per head, lanes over the head dim.  The one score's
+// weight is 2^(s − s) = 1, or NaN for a score that is not finite, as the tiled kernels have
+// it.  Bound by its launch.  32 heads of 128: the 128-row kernel staged a tile of 32 mostly
+// empty keys for it and took 8.1 µs, this takes 2.3.
+__global__ __launch_bounds__(256) void attn_one(AttnArgs g, int heads) {
+    const int bh = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (bh >= heads) return;
+    const int D = g.D, kvh = bh / g.group_size;
+    const float* vrow = g.V + (long long)kvh * D;
+    if (g.v_ld) {
+        const int b = kvh / g.v_heads;
+        vrow = g.V + b * g.v_ld + (long long)(kvh - b * g.v_heads) * D;
+    }
+    const bool in = 4 * lane < D;
+    const int d = in ? 4 * lane : 0;
+    const float4 q = *reinterpret_cast<const float4*>(g.Q + (long long)bh * D + d);
+    const float4 k = *reinterpret_cast<const float4*>(g.K + (long long)kvh * D + d);
+    const float4 v = *reinterpret_cast<const float4*>(vrow + d);
+    const float dot = (q.x * k.x + q.y * k.y) + (q.z * k.z + q.w * k.w);
+    const float sc = wave_sum(in ? dot : 0.f) * g.scale_log2;
+    const float p = __builtin_amdgcn_exp2f(sc - sc);
+    const float w = p / p;
+    // [bh, 1, D] and [B, 1, H, D] are the same rows
+    if (in) *reinterpret_cast<float4*>(g.O + (long long)bh * D + d) = make_float4(v.x * w, v.y * w, v.z * w, v.w * w);
+}
+
+void launch_attn_one(const Step& s, hipStream_t st) {
+    AttnArgs g = make_args(s);
+    if (s.i[12]) {
+        g.v_ld = s.i[12];
+        g.v_heads = (int)s.i[13];
+    }
+    hipLaunchKernelGGL(attn_one, dim3((unsigned)(s.i[0] + 3) / 4), dim3(256), 0, st, g, (int)s.i[0]);
+}
+
 void launch_attn_rows(const Step& s, hipStream_t st) {
     AttnArgs g = make_args(s);
     if (g.S <= 0 || s.i[0] <= 0) return;
@@ -1291,16 +1326,16 @@ void lbr_attn_defer(Step* s) {
 const char* lbr_attn_step_name(const Step& s, bool v, bool t, int store) {
     static const std::vector<std::string> table = [] {
         std::vector<std::string> n;
-        for (int k = 0; k < 2; ++k)
+        for (const char* kernel : {"attn_fwd_mfma16_f32", "attn_fwd_kq_f32", "attn_one_f32"})
             for (int a = 0; a < 2; ++a)
                 for (int b = 0; b < 2; ++b)
                     for (int c = 0; c < 3; ++c)
-                        n.push_back(std::string(k ? "attn_fwd_kq_f32" : "attn_fwd_mfma16_f32") + (a ? "+v" : "") +
+                        n.push_back(std::string(kernel) + (a ? "+v" : "") +
                                     (b ? "+transpose" : "") + (c == 1 ? "+defer" : c == 2 ? "+relay" : ""));
         return n;
     }();
-    const int kq = s.i[15] == 1;
-    return table[(((kq * 2 + (v ? 1 : 0)) * 2 + (t ? 1 : 0)) * 3) + (store < 0 || store > 2 ? 0 : store)].c_str();
+    const int kernel = s.i[17] == 1 ? 2 : s.i[15] == 1 ? 1 : 0;
+    return table[(((kernel * 2 + (v ? 1 : 0)) * 2 + (t ? 1 : 0)) * 3) + (store < 0 || store > 2 ? 0 : store)].c_str();
 }
 
 // Whole heads, or alternate blocks of them, per XCD: the smallest P in
@@ -1440,6 +1475,18 @@ int decode_attention(const OpNode* n, Step* s) {
         // LBR_ATTN_TILE=32 keeps the 32x32 kernel for every head dim (A/B timing).
         const char* tile = getenv("LBR_ATTN_TILE");
         if (dp <= 128 && !(tile && atoi(tile) == 32)) {
+            // One row needs none of the tiled kernels' schedules (8.1 → 2.3 µs, see attn_one), unless
+            // one of them is forced; a mask keeps the tiled kernel, which gives its -inf rows' zeros.
+            const char* const forced[] = {"LBR_ATTN_FOLD", "LBR_ATTN_SPLIT", "LBR_ATTN_SPLIT_WG", "LBR_ATTN_KQ",
+                                          "LBR_ATTN_FOLD64"};
+            if (seq == 1 && !has_mask &&
+                std::none_of(std::begin(forced), std::end(forced), [](const char* e) { return getenv(e); })) {
+                s->run = launch_attn_one;
+                s->name = "attn_one_f32";
+                s->i[17] = 1;
+                s->i[10] = 1;   // writes O as [B, S, H, D] and reads a strided V, like the 16x16 kernel
+                return LBR_OK;
+            }
             // Fold causal query blocks in pairs while that still leaves one
             // 8-wavefront workgroup per CU (LBR_ATTN_FOLD=0/1 overrides).
             const long long nq = (seq + A16_QB - 1) / A16_QB;

@@ -1,11 +1,11 @@
 """A layer on one token: the GEMV's fused epilogues against the node-by-node plan (the same bits) and
-a float64 closed form."""
+a float64 closed form, and the one-row attention against the closed form and the tiled kernel."""
 
 import numpy as np
 import pytest
 
 from conftest import normwise_rel
-from helpers import cf_attention, cf_gelu_tanh, cf_silu, randn, rng
+from helpers import cf_attention, cf_gelu_tanh, cf_silu, one_node_graph, randn, rng, run_gpu
 from runtime.ir import Graph, OpType
 
 pytestmark = pytest.mark.gpu
@@ -90,6 +90,23 @@ def test_gemv_gated(K, F, bias, gbias, order):
     g.add_node(OpType.GATED_ACT, ins, "y", {"has_bias": gbias, "act": "silu"})
     g.outputs.append("y")
     _check(g, {"a": a}, cf_silu(x) * up, "gemv_t+gated")
+
+
+@pytest.mark.parametrize("bh,group,hd,causal", [(32, 4, 128, True), (5, 1, 8, False), (3, 3, 40, True), (1, 1, 64, False)])
+def test_attention_one_row(monkeypatch, bh, group, hd, causal):
+    r = rng(bh + hd)
+    q, k, v = randn(r, 1, bh, 1, hd), randn(r, 1, bh // group, 1, hd), randn(r, 1, bh // group, 1, hd)
+    q[0, 0, 0, 0] = np.inf if bh > 3 else q[0, 0, 0, 0]   # a score that is not finite: the row is NaN
+    attrs = {"causal": causal, **({"group_size": group} if group > 1 else {})}
+    g = one_node_graph(OpType.ATTENTION, {"q": q, "k": k, "v": v}, q.shape, attrs)
+    names = []
+    y = run_gpu(g, {"q": q, "k": k, "v": v}, kernels=names)
+    assert names == ["attn_one_f32"]
+    monkeypatch.setenv("LBR_ATTN_FOLD", "0")
+    np.testing.assert_array_equal(y, run_gpu(g, {"q": q, "k": k, "v": v}))
+    ok = np.isfinite(y)
+    assert ok.all() or bh > 3
+    assert normwise_rel(y[ok], cf_attention(q, k, v, causal=causal, group=group)[ok]) <= 1e-6
 
 
 @pytest.mark.parametrize("H,Hkv,hd,K", [(4, 2, 32, 96), (3, 3, 20, 33)])
