@@ -208,11 +208,12 @@ int lbr_plan_node_kernel(const lbr_plan* plan, int index, char* name_out,
 #define LBR_FUSE_GEMM_HEADS    2  /* MATMUL[_ADD] → k × (SLICE → [ADD bias] → TRANSPOSE(S,H)):
                                      the epilogue writes each column range as [B, H, S, hd]     */
 #define LBR_FUSE_HEAD_PROLOGUE 3  /* SLICE → [ADD bias] → [RMSNORM] → TRANSPOSE(S,H) → [RoPE]
-                                     (7-node rotate-half window) as one kernel                  */
+                                     (7-node rotate-half window, its nodes in any order the data
+                                     allow) as one kernel                                       */
 #define LBR_FUSE_ATTN_TRANSPOSE 4 /* ATTENTION → TRANSPOSE(H,S): the attention kernel writes
                                      its output as [B, S, H, hd]                                */
 #define LBR_FUSE_GEMM_ACT      5  /* MATMUL[_ADD] → RELU | GELU | SILU: the activation is
-                                     applied in the GEMM epilogue                               */
+                                     applied in the GEMM epilogue (one row: the GEMV's)         */
 #define LBR_FUSE_GEMM_GATED    6  /* MATMUL[_ADD] (N = 2F) → SLICE [0,F) → SLICE [F,2F) →
                                      GATED_ACT: the GEMM pairs gate and up columns in each tile
                                      and writes act(gate)·up as [M, F]                           */
@@ -302,6 +303,8 @@ int lbr_attn_kq_grid(long long bh, int seq, int causal, int cus,
  * lbr_plan_step_args reports in [14], less one), "" for other indices: for
  * reports, no counterpart in the reference. */
 const char* lbr_gemm_tile_name(int tile);
+/* 1 for the tiles of the split-bf16 kernel (gemm_split_f32), else 0. */
+int lbr_gemm_tile_split(int tile);
 
 /* The decoded integer launch arguments of step `step` (up to `cap` of them,
  * 40 at most), for tests and reports.  Their meaning is the kernel's: for

@@ -12,8 +12,8 @@
 // a multiple of 32 — all the Linear layers of the workloads — with
 // v_mfma_f32_16x16x4_f32, direct-to-LDS loads and a tile shape chosen per GEMM; of those,
 // gemm_split_f32 (gemm_split.hip) takes the large ones (gemm_family) on the bf16 matrix
-// cores; gemm_mfma_f32 (v_mfma_f32_32x32x2_f32) takes the rest (B stored [K, N], ragged
-// K, unaligned operands).
+// cores, and every K that is a multiple of 4 only; gemm_mfma_f32 (v_mfma_f32_32x32x2_f32)
+// takes the rest (B stored [K, N], other K, unaligned operands).
 //
 // gemm_mfma_f32 tiling: a 256-thread workgroup (4 wavefronts, 2×2) owns a 128×128 tile of
 // C; each wavefront owns 64×64 = 2×2 MFMA blocks of 32×32 (64 accumulator
@@ -1331,6 +1331,10 @@ int gemm_dma_tune_candidates(const Step& s, int* tiles, int cap) {
 
 extern "C" const char* lbr_gemm_tile_name(int tile) {
     return tile >= 0 && tile < kNumDmaTiles ? kDmaTiles[tile].name : "";
+}
+
+extern "C" int lbr_gemm_tile_split(int tile) {
+    return tile >= 0 && tile < kNumDmaTiles && kDmaTiles[tile].family == SPLIT;
 }
 
 int gemm_dma_tile_by_name(const Step& s, const char* name) {

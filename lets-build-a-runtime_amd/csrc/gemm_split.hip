@@ -13,8 +13,9 @@
 //
 // Where the split does not hold, the fp32 matrix cores recompute (fp32_redo): an operand
 // that is infinite, NaN or rounds to an infinite bf16 gives a result that is not finite,
-// and operands so small that m or l are not normal bf16 values give a result below 2⁻⁶⁰;
-// both are seen in the accumulators.
+// and operands so small that the planes lose bits (below 2⁻¹¹⁰; bf16 ends at 2⁻¹³³) give,
+// against operands up to 2⁵⁰, a result below 2⁻⁶⁰; both are seen in the accumulators.
+// Products of values below 2⁻¹¹⁰ with values above 2⁵⁰ keep the planes' fewer bits.
 //
 // Structure: a WGM×WGN grid of wavefronts, each (TM/WGM)×(TN/WGN) of C in 32×32 blocks.  A
 // step is 16 columns of K.  Each thread loads its float4s of the A and B tiles two steps

@@ -289,7 +289,8 @@ class CompiledExecutor(Executor):
             elif d["kernel"].startswith("gemm_"):
                 d.update(m=int(ints[0]), n=int(ints[1]), k=int(ints[2]),
                          tile=lib.lbr_gemm_tile_name(int(ints[14]) - 1).decode() or "legacy",
-                         ksplit=max(1, int(ints[10])), dma_tile=int(ints[14]) - 1, norm=int(ints[15]),
+                         ksplit=max(1, int(ints[10])), dma_tile=int(ints[14]) - 1,
+                         split=bool(lib.lbr_gemm_tile_split(int(ints[14]) - 1)), norm=int(ints[15]),
                          reduce_norm=int(ints[16]), split_for_norm=bool(int(ints[17]) & 256),
                          frag_splits=int(ints[5]) if int(ints[19]) > 0 else 0,
                          head_parts=int(ints[18]))
