@@ -306,13 +306,20 @@ const char* lbr_gemm_tile_name(int tile);
 /* 1 for the tiles of the split-bf16 kernel (gemm_split_f32), else 0. */
 int lbr_gemm_tile_split(int tile);
 
+/* The kernel a MATMUL / MATMUL_ADD node decodes to, unfused: its name, GEMM
+ * tile index (-1: none) and number of K ranges, with 256 CUs taken before
+ * lbr_init: test support, no counterpart in the reference. */
+int lbr_gemm_choice(const OpNode* node, char* name_out, int cap, int* tile,
+                    int* ksplit);
+
 /* The decoded integer launch arguments of step `step` (up to `cap` of them,
- * 40 at most), for tests and reports.  Their meaning is the kernel's: for
+ * 41 at most), for tests and reports.  Their meaning is the kernel's: for
  * the attention kernel [6] = causal blocks folded in pairs, [7] = key-range
  * split workgroups (0: no split), [14] = deferred output, [15] = the
  * key-quartered 16-row kernel; for the GEMM
  * kernels [10] = K ranges, [14] = DMA tile index + 1 (0: register-staged
- * kernel). */
+ * kernel, or with [40] > 0 the split-bf16 kernel's tile index [40] - 1 on a K
+ * that is no multiple of 32). */
 int lbr_plan_step_args(const lbr_plan* plan, int step, long long* ints_out,
                        int cap);
 

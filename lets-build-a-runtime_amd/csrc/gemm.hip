@@ -31,6 +31,7 @@
 // reuse the same A and B panels) hit the same L2.
 #include "gemm_common.h"
 
+#include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <string>
@@ -39,7 +40,8 @@
 //          [7]=sA [8]=sB [9]=sC [10]=ksplit [11]=kchunk [12]=float4 reduce
 //          [13]=1 (takes fused epilogues; 2: gemv_t, which does too) [14]=DMA tile + 1 (0: gemm_mfma_f32)
 //          [19..30] head scatter, [31] activation, [32..34] gated pair, [35..37] A in
-//          head layout (see below) ; f[0] = alpha
+//          head layout (see below), [40]=split-bf16 tile + 1 of a ragged K (whose [14] is 0);
+//          f[0] = alpha
 GemmArgs gemm_make_args(const Step& s) {
     GemmArgs g;
     g.A = (const float*)s.in[0];
@@ -1081,13 +1083,16 @@ double dma_time(const DmaTile& d, long long M, long long N, long long batches, i
 }
 
 // Tile shape and number of K ranges of one family by dma_time.
-// LBR_GEMM_TILE (a tile name) and LBR_GEMM_KSPLIT override the choice.  Returns its time.
+// LBR_GEMM_TILE (a tile name) and LBR_GEMM_KSPLIT override the choice.  Returns its time, or
+// NO_TILE when the overrides leave the family no tile or no such K ranges: the tile is then
+// the fp32 128×128 one with K whole, for callers whose K it takes.
+constexpr double NO_TILE = 1e30;
 double choose_dma(Family family, long long M, long long N, int K, long long batches, int cus, int* tile, int* ksplit,
                   int* kchunk) {
     std::string force_tile;
     forced_tile(&force_tile);
     const char* force_ks = getenv("LBR_GEMM_KSPLIT");
-    double best = 1e30;
+    double best = NO_TILE;
     *tile = 1;
     *ksplit = 1;
     *kchunk = K;
@@ -1474,27 +1479,27 @@ int decode_matmul(const OpNode* n, Step* s) {
     // the register-staged kernel has 128×128 alone (µs, split against register-staged:
     // 231×600×200 9.9 / 20.1, 231×200×712 11.3 / 55, 5×30×20 4.2 / 5.0, 3×1000×4100 15.6 / 30,
     // 1000×4100×2564 145 / 260).  The step keeps the
-    // register-staged kernel's name and epilogues (residual, head scatter).
+    // register-staged kernel's name and epilogues (residual, head scatter).  Overrides that no
+    // split tile meets (a K range count that K does not give, an unknown tile name) leave the
+    // GEMM to the register-staged kernel.
     const bool ragged_split = trans_b && vec && M * K * 4 < (1LL << 31) && (long long)N * K * 4 < (1LL << 31) &&
                               (force_tile || getenv("LBR_GEMM_SPLIT") ? gemm_family(M, N, K, batches) == SPLIT : true);
-    if (ragged_split) {
-        int tile = 0, ks = 1, kchunk = K;
-        choose_dma(SPLIT, M, N, K, batches, lbr_device_cus(), &tile, &ks, &kchunk);
+    int tile = 0, ks = 1, kchunk = K;
+    if (ragged_split &&
+        choose_dma(SPLIT, M, N, K, batches, lbr_device_cus(), &tile, &ks, &kchunk) < NO_TILE) {
         s->i[10] = ks;
         s->i[11] = kchunk;
+        s->i[40] = tile + 1;
         s->ws_bytes = ks > 1 ? (size_t)ks * batches * M * N * sizeof(float) : 0;
         s->run = has_bias ? dma_launcher<true>(tile) : dma_launcher<false>(tile);
         s->name = "gemm_mfma_f32_nt";
         return LBR_OK;
     }
-    {
-        const long long tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN) * batches;
-        int kchunk = K;
-        const int ks = choose_ksplit(tiles, K, M * (long long)N, lbr_device_cus(), &kchunk);
-        s->i[10] = ks;
-        s->i[11] = kchunk;
-        s->ws_bytes = ks > 1 ? (size_t)ks * batches * M * N * sizeof(float) : 0;
-    }
+    const long long tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN) * batches;
+    ks = choose_ksplit(tiles, K, M * (long long)N, lbr_device_cus(), &kchunk);
+    s->i[10] = ks;
+    s->i[11] = kchunk;
+    s->ws_bytes = ks > 1 ? (size_t)ks * batches * M * N * sizeof(float) : 0;
     if (trans_b) {
         if (vec) s->run = has_bias ? launch_gemm_t<true, true, true> : launch_gemm_t<true, true, false>;
         else s->run = has_bias ? launch_gemm_t<true, false, true> : launch_gemm_t<true, false, false>;
@@ -1504,5 +1509,20 @@ int decode_matmul(const OpNode* n, Step* s) {
         else s->run = has_bias ? launch_gemm_t<false, false, true> : launch_gemm_t<false, false, false>;
         s->name = "gemm_mfma_f32_nn";
     }
+    return LBR_OK;
+}
+
+extern "C" int lbr_gemm_choice(const OpNode* node, char* name_out, int cap, int* tile, int* ksplit) {
+    if (!node || !name_out || cap < 1 || !tile || !ksplit ||
+        (node->op != OP_MATMUL && node->op != OP_MATMUL_ADD)) {
+        lbr_set_error("lbr_gemm_choice: bad arguments");
+        return LBR_ERR_INVALID;
+    }
+    if (int rc = lbr_node_check(node, 0)) return rc;
+    Step s = Step();
+    if (int rc = decode_matmul(node, &s)) return rc;
+    snprintf(name_out, cap, "%s", s.name);
+    *tile = (int)(s.i[40] ? s.i[40] : s.i[14]) - 1;
+    *ksplit = std::max(1, (int)s.i[10]);
     return LBR_OK;
 }

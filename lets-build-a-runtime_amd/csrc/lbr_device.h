@@ -330,7 +330,7 @@ struct Step {
     const void* in[MAX_INPUTS];
     void* out;
     int n_in;
-    long long i[40];          // integer parameters (meaning per launcher)
+    long long i[41];          // integer parameters (meaning per launcher)
     float f[4];               // float parameters
     size_t ws_bytes;          // device workspace this step needs (0 = none)
     void* ws;                 // workspace assigned by the plan (shared by all steps)

@@ -85,6 +85,7 @@ class HipLibrary:
             "lbr_fast_div": ([ctypes.c_uint, ctypes.c_uint], ctypes.c_uint),
             "lbr_gemm_tile_name": ([c_int], c_char_p),
             "lbr_gemm_tile_split": ([c_int], c_int),
+            "lbr_gemm_choice": ([P(COpNode), ctypes.c_char_p, c_int, P(c_int), P(c_int)], c_int),
             "lbr_attn_kq_grid": ([ctypes.c_longlong, c_int, c_int, c_int, P(c_int), P(c_int), c_int], c_int),
         }
         for name, (args, res) in sig.items():
@@ -141,6 +142,16 @@ class HipLibrary:
         self.check(self._lib.lbr_check_nodes(nodes, n, int(fuse), lp, lb, len(live), ctypes.byref(steps)),
                    "lbr_check_nodes")
         return steps.value
+
+    def gemm_choice(self, node) -> tuple[str, str, bool, int]:
+        """(kernel name, tile name or "", split-bf16 kernel, K ranges) of an unfused MATMUL /
+        MATMUL_ADD node; needs no device."""
+        name = ctypes.create_string_buffer(64)
+        tile, ks = ctypes.c_int(), ctypes.c_int()
+        self.check(self._lib.lbr_gemm_choice(ctypes.byref(node), name, 64, ctypes.byref(tile), ctypes.byref(ks)),
+                   "lbr_gemm_choice")
+        return (name.value.decode(), self._lib.lbr_gemm_tile_name(tile.value).decode(),
+                bool(self._lib.lbr_gemm_tile_split(tile.value)), ks.value)
 
 
 def live_arrays(live: list[tuple[int, int]]):

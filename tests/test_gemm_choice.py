@@ -1,0 +1,41 @@
+"""The kernel a MATMUL node takes, on the CPU (lbr_gemm_choice: nothing is launched)."""
+
+import pytest
+
+from runtime.ir import OpType
+from test_fusion import _lib, _node
+
+BASE = 1 << 40
+
+
+def _choice(M, N, K, batches=1, trans_b=1):
+    shape = (1, M, N) if batches == 1 else (batches, M, N)
+    return _lib().gemm_choice(_node(OpType.MATMUL, [BASE, 2 * BASE], 3 * BASE, shape,
+                                    (K, trans_b, int(batches == 1), 0)))
+
+
+@pytest.fixture(autouse=True)
+def _no_overrides(monkeypatch):
+    for e in ("LBR_GEMM_TILE", "LBR_GEMM_KSPLIT", "LBR_GEMM_SPLIT"):
+        monkeypatch.delenv(e, raising=False)
+
+
+@pytest.mark.parametrize("K,ks", [(20, 2), (20, 16), (200, 5), (200, 6), (712, 16), (1036, 16)])
+def test_ragged_k_with_ranges_it_does_not_give(monkeypatch, K, ks):
+    """A K that does not cut into the forced number of whole 32-wide ranges has no split tile: the
+    register-staged kernel runs, never an fp32 DMA tile, which would drop the columns past K/32·32."""
+    monkeypatch.setenv("LBR_GEMM_KSPLIT", str(ks))
+    assert _choice(300, 70, K)[:3] == ("gemm_mfma_f32_nt", "", False)
+
+
+def test_ragged_k_with_a_tile_the_split_kernel_lacks(monkeypatch):
+    for name in ("32x48b3", "nonsenseb3", "b3"):
+        monkeypatch.setenv("LBR_GEMM_TILE", name)
+        assert _choice(300, 70, 200)[:3] == ("gemm_mfma_f32_nt", "", False), name
+
+
+@pytest.mark.parametrize("K,ks", [(712, 2), (712, 3), (100, 4), (1036, 11)])
+def test_ragged_k_with_ranges_it_gives(monkeypatch, K, ks):
+    monkeypatch.setenv("LBR_GEMM_KSPLIT", str(ks))
+    name, tile, split, got = _choice(300, 70, K)
+    assert name == "gemm_mfma_f32_nt" and tile and split and got == ks

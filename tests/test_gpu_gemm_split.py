@@ -54,6 +54,14 @@ def test_split_ragged_k(monkeypatch, tile, M, N, K, batches):
     assert _gemm_case(M, N, K, True, batches, batches == 1, True) == "gemm_mfma_f32_nt"
 
 
+@pytest.mark.parametrize("K", [20, 200, 712])
+@pytest.mark.parametrize("ks", [2, 6, 16])
+def test_ragged_k_under_forced_ranges(monkeypatch, K, ks):
+    """Every column of a ragged K counts, whether K gives that many ranges or not."""
+    monkeypatch.setenv("LBR_GEMM_KSPLIT", str(ks))
+    _gemm_case(300, 70, K, True, 1, True, False)
+
+
 def _run(a, b):
     M, K = a.shape
     g = one_node_graph(OpType.MATMUL, {"a": a[None]}, (1, M, b.shape[0]), {"transpose_b": True}, {"b": b})
