@@ -11,11 +11,16 @@
 // kernel's at every K (N(0,1) rows: 1.1e-7 / 4.2e-7 / 9.8e-7 at K = 64 / 768 / 4096 against
 // 1.4e-7 / 5.0e-7 / 1.15e-6; GELU outputs at K = 16384: 1.8e-6 against 2.3e-6).
 //
-// Where the split does not hold, the fp32 matrix cores recompute (fp32_redo): an operand
-// that is infinite, NaN or rounds to an infinite bf16 gives a result that is not finite,
-// and operands so small that the planes lose bits (below 2⁻¹¹⁰; bf16 ends at 2⁻¹³³) give,
-// against operands up to 2⁵⁰, a result below 2⁻⁶⁰; both are seen in the accumulators.
-// Products of values below 2⁻¹¹⁰ with values above 2⁵⁰ keep the planes' fewer bits.
+// Range: both operands are taken times 2²⁴ and the sum times 2⁻⁴⁸, all exact, so that the
+// planes of every finite value below 2¹⁰⁴, subnormals included, are zero or normal bf16
+// values (the smallest fp32 bit, 2⁻¹⁴⁹, becomes 2⁻¹²⁵) and no bit is lost.  Operands from
+// 2¹⁰⁴ up, infinities and NaN, and sums from 2⁸⁰ up give an accumulator that is not finite,
+// and the fp32 matrix cores recompute the 32×32 blocks that hold one.  Unscaled planes lost
+// bits below 2⁻¹¹⁰ and all of them below 2⁻¹³⁴.  The scaling takes the place of the sign's
+// XOR on A and costs B a multiplication an element: 1% of 4096×12288×4096 on 256×256 tiles
+// (1776 → 1783 µs) and 3% of 1024×6144×2560 on 64×128, which steps in pairs (below) win back
+// (1762, and 201 against 202).  A block that is recomputed reads its rows of A and B from
+// memory for itself: a product with such values everywhere runs at a fraction of the rate.
 //
 // Structure: a WGM×WGN grid of wavefronts, each (TM/WGM)×(TN/WGN) of C in 32×32 blocks.  A
 // step is 16 columns of K.  Each thread loads its float4s of the A and B tiles two steps
@@ -34,8 +39,7 @@
 // that and the loads the rest.
 #include "gemm_common.h"
 
-#include <cstdlib>
-#include <cstring>
+#include <type_traits>
 
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -51,19 +55,17 @@ __device__ __forceinline__ unsigned cvt_bf16x2(float a, float b) {
 // The planes of two neighbours, packed: x = h + m + l exactly (l fits: after two
 // round-to-nearest steps at most 8 significant bits are left).
 __device__ __forceinline__ void split3(float x0, float x1, unsigned& h, unsigned& m, unsigned& l) {
+#pragma clang fp contract(off)   // a subtraction is the shorter instruction
     h = cvt_bf16x2(x0, x1);
     const float r0 = x0 - __uint_as_float(h << 16), r1 = x1 - __uint_as_float(h & 0xffff0000u);
     m = cvt_bf16x2(r0, r1);
     l = cvt_bf16x2(r0 - __uint_as_float(m << 16), r1 - __uint_as_float(m & 0xffff0000u));
 }
 
-// Whether an accumulator is outside what the split vouches for: not finite, or nonzero and
-// below 2⁻⁶⁰.
-__device__ __forceinline__ bool outside_split(float v) {
-    constexpr unsigned LOW = 0x21800000u;   // 2⁻⁶⁰
-    const unsigned u = __float_as_uint(v) & 0x7fffffffu;
-    return u - LOW >= 0x7f800000u - LOW && u != 0;
-}
+// Powers of two that keep the planes of subnormal operands normal (see the top).
+constexpr float UP = 0x1p24f, DOWN = 0x1p-48f;
+
+__device__ __forceinline__ bool not_finite(float v) { return (__float_as_uint(v) & 0x7fffffffu) >= 0x7f800000u; }
 
 // The bf16 MFMAs round their fp32 sum down, not to nearest: 4096 terms of N(0,1) rows came
 // out 2.1e-7 of their rms too low on average, which an average over many of them (attention
@@ -78,6 +80,10 @@ template <int TM, int TN, int WGM, int WGN, int OCC, bool HAS_BIAS, bool AHEADS,
 __global__ __launch_bounds__(64 * WGM * WGN, OCC) void gemm_split_f32(GemmArgs g) {
     constexpr int NT = 64 * WGM * WGN;
     constexpr int WM = TM / WGM, WN = TN / WGN, FM = WM / 32, FN = WN / 32;
+    // One MFMA block a wavefront: a step is a chain of latencies, which wants fewer VALU
+    // instructions between the MFMAs and, with the ragged tail's selects, no steps in pairs
+    // (231×200×712: 21.2 µs against 23.0 with both as on the other tiles).
+    constexpr bool ONE = FM * FN == 1;
     constexpr int KB = 16, QR = KB / 4;                       // float4s ("quads") per tile row and step
     constexpr int NA = TM * QR / NT, NB = TN * QR / NT, NQ = NA + NB;   // quads per thread
     static_assert(NA * NT == TM * QR && NB * NT == TN * QR, "tile rows must split evenly over the threads");
@@ -138,13 +144,10 @@ __global__ __launch_bounds__(64 * WGM * WGN, OCC) void gemm_split_f32(GemmArgs g
         raw[t] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(t < NA ? ra : rb, o, so, 0));
     };
     unsigned ph[2], pm[2], pl[2];
-    auto split = [&](int p, unsigned sign) {   // pair p: components 2·(p&1), 2·(p&1)+1 of quad p/2
-        float x0 = raw[p >> 1][2 * (p & 1)], x1 = raw[p >> 1][2 * (p & 1) + 1];
-        if ((p >> 1) < NA) {   // A's sign is the group's (see GROUP)
-            x0 = __uint_as_float(__float_as_uint(x0) ^ sign);
-            x1 = __uint_as_float(__float_as_uint(x1) ^ sign);
-        }
-        split3(x0, x1, ph[p & 1], pm[p & 1], pl[p & 1]);
+    auto split = [&](int p, float up) {   // pair p: components 2·(p&1), 2·(p&1)+1 of quad p/2
+#pragma clang fp contract(off)
+        const float f = (p >> 1) < NA ? up : UP;   // A's sign is the group's (see GROUP)
+        split3(raw[p >> 1][2 * (p & 1)] * f, raw[p >> 1][2 * (p & 1) + 1] * f, ph[p & 1], pm[p & 1], pl[p & 1]);
     };
     auto negate = [&](auto& a) {
 #pragma unroll
@@ -196,54 +199,66 @@ __global__ __launch_bounds__(64 * WGM * WGN, OCC) void gemm_split_f32(GemmArgs g
         for (int t = 0; t < NQ; ++t) load(t, kbeg);
 #pragma unroll
         for (int t = 0; t < NQ; ++t) {
-            split(2 * t, 0u);
-            split(2 * t + 1, 0u);
+            split(2 * t, UP);
+            split(2 * t + 1, UP);
             put(lds, t);
             load(t, kbeg + min(1, nk - 1) * KB);
         }
         __syncthreads();
-        int cur = 0;
+        // one step; CUR (0 or STAGE): where its planes are, the other stage takes the next step's
+        auto step = [&](int kt, auto CUR) {
+            // steps past the last are re-fetches of the last one, into a stage nothing reads
+            const char* st = lds + CUR;
+            char* wr = lds + (STAGE - CUR);
+            const int k2 = kbeg + min(kt + 2, nk - 1) * KB;
+            // of the step being split: UP, negative in every other group
+            const float up = __uint_as_float(__float_as_uint(UP) | (unsigned)((kt + 1) / GROUP & 1) << 31);
+            get_a(st);
+            get_b(st, 0, fb[0]);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int j = 0; j < FN; ++j) {
+                constexpr int NP = 2 * NQ, VPM = ((NP + FN - 1) / FN * (ONE ? 9 : 13) + 6 * FM - 1) / (6 * FM);
+                if (j + 1 < FN) get_b(st, j + 1, fb[(j + 1) & 1]);
+                mma(j, fb[j & 1]);
+#pragma unroll
+                for (int p = 0; p < NP; ++p)   // this block's share of the next step's pairs
+                    if (p * FN / NP == j) {
+                        split(p, up);
+                        if (p & 1) {
+                            put(wr, p >> 1);
+                            load(p >> 1, k2);
+                        }
+                    }
+                if (j + 1 < FN) __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);   // the fragment reads first
+#pragma unroll
+                for (int q = 0; q < 6 * FM; ++q) {   // then each MFMA with its share of the splitting
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x002, VPM, 0);
+                }
+                if (j + 1 < FN) __builtin_amdgcn_sched_barrier(0);
+            }
+            __syncthreads();
+        };
         for (int k0 = 0; k0 < nk; k0 += GROUP) {
             if (k0) negate(acc);
-            for (int kt = k0; kt < min(nk, k0 + GROUP); ++kt) {
-                // steps past the last are re-fetches of the last one, into a stage nothing reads
-                const char* st = lds + cur;
-                char* wr = lds + (STAGE - cur);
-                const int k2 = kbeg + min(kt + 2, nk - 1) * KB;
-                const unsigned sign = ((kt + 1) / GROUP & 1) ? 0x80000000u : 0u;   // of the step being split
-                get_a(st);
-                get_b(st, 0, fb[0]);
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int j = 0; j < FN; ++j) {
-                    constexpr int NP = 2 * NQ, VPM = ((NP + FN - 1) / FN * 11 + 6 * FM - 1) / (6 * FM);
-                    if (j + 1 < FN) get_b(st, j + 1, fb[(j + 1) & 1]);
-                    mma(j, fb[j & 1]);
-#pragma unroll
-                    for (int p = 0; p < NP; ++p)   // this block's share of the next step's pairs
-                        if (p * FN / NP == j) {
-                            split(p, sign);
-                            if (p & 1) {
-                                put(wr, p >> 1);
-                                load(p >> 1, k2);
-                            }
-                        }
-                    if (j + 1 < FN) __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);   // the fragment reads first
-#pragma unroll
-                    for (int q = 0; q < 6 * FM; ++q) {   // then each MFMA with its share of the splitting
-                        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                        __builtin_amdgcn_sched_group_barrier(0x002, VPM, 0);
-                    }
-                    if (j + 1 < FN) __builtin_amdgcn_sched_barrier(0);
+            const int kl = min(nk, k0 + GROUP);
+            int kt = k0;
+            if constexpr (!(ONE && RAGGED))
+                for (; kt + 1 < kl; kt += 2) {   // in pairs: the stages' addresses are constants
+                    step(kt, std::integral_constant<int, 0>());
+                    step(kt + 1, std::integral_constant<int, STAGE>());
                 }
-                __syncthreads();
-                cur = STAGE - cur;
-            }
+            for (; kt < kl; ++kt) step(kt, (kt & 1) * STAGE);
         }
-        if ((nk - 1) / GROUP & 1) negate(acc);
+        const float down = ((nk - 1) / GROUP & 1) ? -DOWN : DOWN;
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j) acc[i][j] = acc[i][j] * down;
     }
 
-    // Blocks with a result the split does not vouch for: the whole block again on the fp32
+    // Blocks with a sum that is not finite: the whole block again on the fp32
     // matrix cores, fragments straight from memory (lane (fh, fr) reads 4 consecutive k of
     // its row, MFMA q takes k = 4·fh + q of an 8-wide chunk), and those results replaced.
 #pragma unroll
@@ -252,7 +267,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, OCC) void gemm_split_f32(GemmArgs g
         for (int j = 0; j < FN; ++j) {
             bool bad = false;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) bad = bad || outside_split(acc[i][j][r]);
+            for (int r = 0; r < 16; ++r) bad = bad || not_finite(acc[i][j][r]);
             if (!__any(bad)) continue;
             const unsigned oa = (unsigned)a_row(m0 + wm * WM + i * 32 + fr) * 4u;
             const unsigned ob = (unsigned)b_row(wn * WN + j * 32 + fr) * 4u;
@@ -271,7 +286,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, OCC) void gemm_split_f32(GemmArgs g
             }
 #pragma unroll
             for (int r = 0; r < 16; ++r)
-                if (outside_split(acc[i][j][r])) acc[i][j][r] = f[r];
+                if (not_finite(acc[i][j][r])) acc[i][j][r] = f[r];
         }
 
     gemm_epilogue<TM, TN, WGM, WGN, 32, HAS_BIAS, !AHEADS, 2 * STAGE / 4>(g, reinterpret_cast<float*>(lds), acc, m0, n0,

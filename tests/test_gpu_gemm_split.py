@@ -1,5 +1,6 @@
 """The split-bf16 GEMM (gemm_split.hip): every tile at its edges against a float64 closed form, its
-epilogues, and the results it hands to the fp32 matrix cores (infinities, NaN, tiny operands).
+epilogues, operands of every exponent, and the results it hands to the fp32 matrix cores (infinities,
+NaN, the largest values).
 
 The tolerance is the fp32 kernel's own: a dot product of K terms summed in fp32 is off by at most
 about K·2⁻²⁴ of Σ|a·b|; for the N(0,1) operands here that is below 1e-5 of the largest result."""
@@ -79,8 +80,8 @@ def test_split_is_exact_where_fp32_is(monkeypatch, tile):
 
 @pytest.mark.parametrize("tile", ["256x256b3", "64x64b3"])
 def test_split_outside_range(monkeypatch, tile):
-    """Infinities, NaN, the largest finite values (infinite as bf16) and tiny operands (whose
-    low planes are no normal bf16 values) give what the fp32 kernel gives."""
+    """Infinities, NaN, the largest finite values (infinite as scaled bf16) and tiny operands (whose
+    low planes, unscaled, are no normal bf16 values) give what the fp32 kernel gives."""
     monkeypatch.setenv("LBR_GEMM_KSPLIT", "1")
     r = rng(11)
     a, b = randn(r, 200, 96), randn(r, 150, 96)
@@ -107,3 +108,24 @@ def test_split_outside_range(monkeypatch, tile):
     for rows in ([100], [101], [102], [0, 1, 2, 60, 199]):   # each range by its own size
         ok = np.isfinite(y[rows])
         assert normwise_rel(x[rows][ok], ref[rows][ok]) <= 1e-5
+
+
+@pytest.mark.parametrize("tile", ["256x256b3", "64x64b3"])
+def test_split_operand_range(monkeypatch, tile):
+    """Operands of every exponent, subnormals included, against small and large ones: no bit of an
+    operand is lost.  Bound: 6 roundings down (2⁻²³ of the partial sum each) per 16 terms, and the
+    products left out (2⁻²⁴ of a product); results below the fp32 range to its last bit."""
+    monkeypatch.setenv("LBR_GEMM_TILE", tile)
+    monkeypatch.setenv("LBR_GEMM_KSPLIT", "1")
+    r, K = rng(21), 96
+    ea = np.repeat([-145, -140, -136, -134, -130, -125, -120, -111, -100, -60, 0, 60, 100, 120], 5)
+    eb = np.repeat([-140, -120, -60, 0, 15, 40, 50, 51, 80, 100, 110, 122], 11)
+    a, b = (np.ldexp(r.standard_normal((len(e), K)), e[:, None]).astype(np.float32) for e in (ea, eb))
+    y = _run(a, b).astype(np.float64)
+    a, b = a.astype(np.float64), b.astype(np.float64)
+    ref, size = a @ b.T, np.abs(a) @ np.abs(b).T
+    tol = (6 * K / 16 + 1) * 2.0 ** -23 * size + K * 2.0 ** -149
+    fits = size < 2.0 ** 127
+    assert fits.sum() > 8000
+    bad = fits & ~(np.abs(y - ref) <= tol)
+    assert not bad.any(), sorted({(int(ea[i]), int(eb[j])) for i, j in zip(*np.nonzero(bad))})
