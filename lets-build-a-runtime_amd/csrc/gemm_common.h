@@ -67,6 +67,7 @@ struct GemmArgs {
     const float* nt_w;
     const float* nt_b;
     float nt_eps;
+    int group;                // split-bf16 kernel: K steps between changes of the sum's sign
 };
 
 // Final store of one C element (row m, column n of batch bz) with the fused

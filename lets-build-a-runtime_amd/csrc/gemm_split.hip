@@ -69,10 +69,17 @@ __device__ __forceinline__ bool not_finite(float v) { return (__float_as_uint(v)
 
 // The bf16 MFMAs round their fp32 sum down, not to nearest: 4096 terms of N(0,1) rows came
 // out 2.1e-7 of their rms too low on average, which an average over many of them (attention
-// over its keys) would keep.  So the sum changes sign every GROUP steps, accumulators and A
-// alike, and the half of it that is negated rounds up: 9e-9 at the same size, at no
-// measurable cost (1723 µs against 1730 for 4096×12288×4096).
+// over its keys) would keep.  So the sum changes sign, accumulators and A alike, between
+// groups of at most GROUP steps, an even number of about equal size (even themselves: the
+// steps go in pairs), and the half of it that is negated rounds up.  Mean error of 512×512
+// results in their rms, N(0,1) rows: -5e-10 / -3e-9 / 2e-9 / 1e-8 at K = 128 / 200 / 256 / 4096,
+// against -9e-9 / -1.3e-8 / -1.5e-8 / -2.1e-7 where it does not change.  Two steps or less stay
+// one group (-8e-9 at K = 16, of an error of 3.4e-8; the fp32 kernels' is 7.4e-8).
 constexpr int GROUP = 16;
+int sign_group(int nk) {   // steps a group, of nk
+    const int n = (nk + 2 * GROUP - 1) / (2 * GROUP) * 2;   // groups
+    return ((nk + n - 1) / n + 1) & ~1;
+}
 
 // K: any multiple of 4 with RAGGED (the last step's columns past K read as zero through
 // the buffer views' range check), else a multiple of 16.
@@ -82,7 +89,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, OCC) void gemm_split_f32(GemmArgs g
     constexpr int WM = TM / WGM, WN = TN / WGN, FM = WM / 32, FN = WN / 32;
     // One MFMA block a wavefront: a step is a chain of latencies, which wants fewer VALU
     // instructions between the MFMAs and, with the ragged tail's selects, no steps in pairs
-    // (231×200×712: 21.2 µs against 23.0 with both as on the other tiles).
+    // (231×200×712: 21.7 µs against 23.0 with both as on the other tiles).
     constexpr bool ONE = FM * FN == 1;
     constexpr int KB = 16, QR = KB / 4;                       // float4s ("quads") per tile row and step
     constexpr int NA = TM * QR / NT, NB = TN * QR / NT, NQ = NA + NB;   // quads per thread
@@ -206,13 +213,13 @@ __global__ __launch_bounds__(64 * WGM * WGN, OCC) void gemm_split_f32(GemmArgs g
         }
         __syncthreads();
         // one step; CUR (0 or STAGE): where its planes are, the other stage takes the next step's
-        auto step = [&](int kt, auto CUR) {
+        auto step = [&](int kt, int kl, bool pos, auto CUR) {
             // steps past the last are re-fetches of the last one, into a stage nothing reads
             const char* st = lds + CUR;
             char* wr = lds + (STAGE - CUR);
             const int k2 = kbeg + min(kt + 2, nk - 1) * KB;
             // of the step being split: UP, negative in every other group
-            const float up = __uint_as_float(__float_as_uint(UP) | (unsigned)((kt + 1) / GROUP & 1) << 31);
+            const float up = (kt + 1 < kl) == pos ? UP : -UP;
             get_a(st);
             get_b(st, 0, fb[0]);
             __builtin_amdgcn_sched_barrier(0);
@@ -240,18 +247,21 @@ __global__ __launch_bounds__(64 * WGM * WGN, OCC) void gemm_split_f32(GemmArgs g
             }
             __syncthreads();
         };
-        for (int k0 = 0; k0 < nk; k0 += GROUP) {
-            if (k0) negate(acc);
-            const int kl = min(nk, k0 + GROUP);
-            int kt = k0;
+        bool pos = true;
+        for (int kt = 0; kt < nk;) {
+            const int kl = min(nk, kt + g.group);
             if constexpr (!(ONE && RAGGED))
                 for (; kt + 1 < kl; kt += 2) {   // in pairs: the stages' addresses are constants
-                    step(kt, std::integral_constant<int, 0>());
-                    step(kt + 1, std::integral_constant<int, STAGE>());
+                    step(kt, kl, pos, std::integral_constant<int, 0>());
+                    step(kt + 1, kl, pos, std::integral_constant<int, STAGE>());
                 }
-            for (; kt < kl; ++kt) step(kt, (kt & 1) * STAGE);
+            for (; kt < kl; ++kt) step(kt, kl, pos, (kt & 1) * STAGE);
+            if (kt < nk) {
+                negate(acc);
+                pos = !pos;
+            }
         }
-        const float down = ((nk - 1) / GROUP & 1) ? -DOWN : DOWN;
+        const float down = pos ? DOWN : -DOWN;
 #pragma unroll
         for (int i = 0; i < FM; ++i)
 #pragma unroll
@@ -299,6 +309,7 @@ void launch(const Step& s, hipStream_t st) {
     if (g.M <= 0 || g.N <= 0) return;
     g.tiles_m = (g.M + TM - 1) / TM;
     g.tiles_n = g.gF ? (g.gF + TN / 2 - 1) / (TN / 2) : (g.N + TN - 1) / TN;
+    g.group = sign_group((g.kchunk + 15) / 16);
     const dim3 grid(g.tiles_m * g.tiles_n, g.ksplit, (unsigned)s.i[3]);
     if (g.K % 16 == 0)
         hipLaunchKernelGGL((gemm_split_f32<TM, TN, WGM, WGN, OCC, HAS_BIAS, AHEADS, false>), grid,

@@ -129,3 +129,18 @@ def test_split_operand_range(monkeypatch, tile):
     assert fits.sum() > 8000
     bad = fits & ~(np.abs(y - ref) <= tol)
     assert not bad.any(), sorted({(int(ea[i]), int(eb[j])) for i, j in zip(*np.nonzero(bad))})
+
+
+@pytest.mark.parametrize("K", [64, 128, 200, 256])
+def test_split_mean_error_of_short_k(monkeypatch, K):
+    """The sum changes sign within a short K too, so that its roundings down do not add up: the mean
+    error of 512x512 results, whose own spread is 2.4e-7 / 512 = 5e-10 of their rms, is within 7e-9 of
+    it (one sign throughout gives 7e-9 at K = 64, 1.3e-8 at 200, 1.5e-8 at 256)."""
+    monkeypatch.setenv("LBR_GEMM_TILE", "64x64b3")
+    monkeypatch.setenv("LBR_GEMM_KSPLIT", "1")
+    r = rng(K)
+    a, b = randn(r, 512, K), randn(r, 512, K)
+    ref = a.astype(np.float64) @ b.T.astype(np.float64)
+    err, rms = _run(a, b) - ref, np.sqrt((ref ** 2).mean())
+    assert abs(err.mean()) <= 7e-9 * rms
+    assert np.sqrt((err ** 2).mean()) <= 3e-7 * rms
