@@ -751,6 +751,7 @@ __device__ __forceinline__ void gemv_rows(const float* __restrict__ a, const flo
 
 template <bool VEC, bool HAS_BIAS>
 __global__ __launch_bounds__(256) void gemv_t(GemmArgs g) {
+#pragma clang fp contract(off)   // alpha·acc + resid is two roundings, as the unfused nodes' (splitk_reduce)
     const int lane = threadIdx.x & 63;
     const int n = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (n >= g.N) return;
@@ -764,6 +765,7 @@ __global__ __launch_bounds__(256) void gemv_t(GemmArgs g) {
 // Gated pair: out[j] = act(gate[j] (+ gated bias))·up[j], rounded as the unfused nodes would.
 template <bool VEC, bool HAS_BIAS>
 __global__ __launch_bounds__(256) void gemv_t_gated(GemmArgs g) {
+#pragma clang fp contract(off)
     const int lane = threadIdx.x & 63;
     const int o = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (o >= g.gF) return;

@@ -12,6 +12,7 @@ pytestmark = pytest.mark.gpu
 
 
 def _gemv(K, N, bias, r):
+    """A one-row MATMUL_ADD, or without `bias` a MATMUL with an alpha that is no power of two."""
     g = Graph()
     a, w = randn(r, 1, 1, K), randn(r, N, K, scale=0.1)
     g.add_tensor("a", (1, 1, K))
@@ -24,8 +25,11 @@ def _gemv(K, N, bias, r):
         g.add_tensor("b", (N,)).buffer = b
         g.constants.append("b")
         ins, c = ins + ["b"], c + b
+    else:
+        c = c * 0.3
     g.add_tensor("c", (1, 1, N))
-    g.add_node(OpType.MATMUL_ADD if bias else OpType.MATMUL, ins, "c", {"transpose_b": True})
+    g.add_node(OpType.MATMUL_ADD if bias else OpType.MATMUL, ins, "c",
+               {"transpose_b": True, **({} if bias else {"alpha": 0.3})})
     return g, a, c
 
 
@@ -46,7 +50,7 @@ def _check(g, feed, ref, name):
     assert normwise_rel(ys[0], ref) <= 1e-5
 
 
-@pytest.mark.parametrize("K,N,bias", [(256, 130, True), (33, 7, False), (2560, 4, True)])
+@pytest.mark.parametrize("K,N,bias", [(256, 130, True), (33, 7, False), (2560, 4, True), (256, 1000, False)])
 def test_gemv_residual(K, N, bias):
     r = rng(K + N)
     g, a, c = _gemv(K, N, bias, r)
