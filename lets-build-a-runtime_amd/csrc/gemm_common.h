@@ -280,28 +280,57 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, float* lds, con
         return;
     }
     float* __restrict__ C = g.C + bz * g.sC;
-    const float* __restrict__ R = g.resid ? g.resid + bz * g.sC : nullptr;
+    if (g.resid) {   // never with a fused activation
+        // As many residual loads as 16 registers (or one block column) hold go out before the
+        // first store, rows and columns clamped, not skipped: a load that follows a store waits
+        // for it.  Two 333-token sequences of width 768, masked attention layer (64×64 fp32
+        // tiles): 77.1 µs, against 77.8 with four loads at a time, 78.9 with loads skipped.
+#pragma clang fp contract(off)   // as the unfused nodes round
+        const float* __restrict__ R = g.resid + bz * g.sC;
+        constexpr int JC = std::clamp(4 / RG, 1, CG);   // block columns at a time
+#pragma unroll
+        for (int j0 = 0; j0 < CG; j0 += JC) {
+            float rv[JC][RG][4];
+#pragma unroll
+            for (int j = 0; j < JC && j0 + j < CG; ++j) {
+                const int n = min(nw + (j0 + j) * CB + cl, N - 1);
+#pragma unroll
+                for (int i = 0; i < RG; ++i)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) rv[j][i][r] = R[(long long)min(mw + i * RS + r, M - 1) * N + n];
+            }
+#pragma unroll
+            for (int j = 0; j < JC && j0 + j < CG; ++j) {
+                const int n = nw + (j0 + j) * CB + cl;
+                if (n >= N) continue;
+                const float bv = HAS_BIAS ? bias[n] : 0.f;
+#pragma unroll
+                for (int i = 0; i < RG; ++i)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int m = mw + i * RS + r;
+                        if (m >= M) continue;
+                        const float v = HAS_BIAS ? (acc_at(acc, i, j0 + j, r) + bv) : alpha * acc_at(acc, i, j0 + j, r);
+                        C[(long long)m * N + n] = v + rv[j][i][r];
+                    }
+            }
+        }
+        return;
+    }
 #pragma unroll
     for (int j = 0; j < CG; ++j) {
         const int n = nw + j * CB + cl;
         if (n >= N) continue;
         const float bv = HAS_BIAS ? bias[n] : 0.f;
 #pragma unroll
-        for (int i = 0; i < RG; ++i) {
-            float rv[4] = {0.f, 0.f, 0.f, 0.f};
-            if (R) {   // rows clamped, not skipped: the four loads go out together
-#pragma unroll
-                for (int r = 0; r < 4; ++r) rv[r] = R[(long long)min(mw + i * RS + r, M - 1) * N + n];
-            }
+        for (int i = 0; i < RG; ++i)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int m = mw + i * RS + r;
                 if (m >= M) continue;
-                float v = HAS_BIAS ? (acc_at(acc, i, j, r) + bv) : alpha * acc_at(acc, i, j, r);
-                if (R) v = v + rv[r];
-                C[(long long)m * N + n] = lbr_act(act, v);   // a fused activation never comes with resid
+                const float v = HAS_BIAS ? (acc_at(acc, i, j, r) + bv) : alpha * acc_at(acc, i, j, r);
+                C[(long long)m * N + n] = lbr_act(act, v);
             }
-        }
     }
 }
 
