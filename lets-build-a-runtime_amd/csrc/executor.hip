@@ -449,11 +449,13 @@ static bool bad_live(const void* const* live_ptr, const size_t* live_bytes, int 
 // than the model's.  A listed step (same step name and M, N, K) takes its
 // tile, and its number of K ranges when `ks` > 0, without timing, so plans
 // come out the same run to run; the model's pick holds for every other step.
-// Every tile sums each output's K terms in the same order: the tile never
-// changes a result bit; another number of K ranges sums the ranges' partial
-// sums instead (a step whose reduce carries a norm keeps its ranges).
+// Every tile of a family sums each output's K terms in the same order: the tile
+// never changes a result bit; another number of K ranges sums the ranges' partial
+// sums instead (a step whose reduce carries a norm keeps its ranges).  A size listed
+// for every step (step null) also takes the fp32 family where gemm_family would send
+// it to the split-bf16 kernel.
 struct TunedTile {
-    const char* step;
+    const char* step;   // null: every step of the size
     long long M, N, K;
     const char* tile;
     int ks;   // K ranges; 0: the step's own
@@ -466,10 +468,18 @@ static const TunedTile kTunedTiles[] = {
     {"gemm_dma_f32_nt+act", 512, 3072, 768, "32x64", 0},         // FFN1: 25.6 against 27.5 (32x48)
     {"gemm_dma_f32_nt+resid", 512, 768, 3072, "32x96", 2},       // FFN2: 28.2 against 30.4 (64x64, 8 ranges)
     // GPT-2 body and LM (1024 rows)
-    {"gemm_dma_f32_nt+heads", 1024, 2304, 768, "32x96", 0},      // QKV: 34.9 against 43.3 (32x48s4)
+    // QKV: 34.3-35.1 in the body's plan, against 37.3 split (64x64b3); 37.3 for a single replayed
+    // node, against 41.2 split and 45.9 on the model's fp32 64x64
+    {nullptr, 1024, 2304, 768, "32x96", 0},
     {"gemm_dma_f32_nt+resid+layernorm", 1024, 768, 768, "32x96", 0},   // O proj + LN: 19.6 against 22.2
     {"gemm_dma_f32_nt+resid", 1024, 768, 768, "32x96", 1},       // O proj (LM): 15.0 against 18.0 (64x64)
 };
+
+bool lbr_tuned_fp32_size(long long M, long long N, long long K) {
+    for (const TunedTile& t : kTunedTiles)
+        if (!t.step && M == t.M && N == t.N && K == t.K) return true;
+    return false;
+}
 
 // The tiles (and K ranges) of kTunedTiles, before the plan's workspace is
 // sized; marks the steps it set.  Skipped under LBR_GEMM_AUTOTUNE=0 or 2 and
@@ -483,7 +493,7 @@ static void table_tiles(std::vector<Step>& steps, std::vector<char>* tabled) {
         Step& s = steps[i];
         if (!s.name || strncmp(s.name, "gemm_dma_f32", 12) != 0 || !s.i[14] || s.i[3] != 1) continue;
         for (const TunedTile& t : kTunedTiles) {
-            if (strcmp(s.name, t.step) != 0 || s.i[0] != t.M || s.i[1] != t.N || s.i[2] != t.K) continue;
+            if ((t.step && strcmp(s.name, t.step) != 0) || s.i[0] != t.M || s.i[1] != t.N || s.i[2] != t.K) continue;
             const int tile = gemm_dma_tile_by_name(s, t.tile);
             Step u = s;
             if (tile < 0 || !gemm_dma_retile(&u, tile) || (t.ks > 0 && !gemm_dma_set_ksplit(&u, t.ks))) continue;

@@ -1129,10 +1129,12 @@ double choose_dma(Family family, long long M, long long N, int K, long long batc
     return best;
 }
 
-// The family of a GEMM: the split-bf16 kernel from 1.5e9 multiply-adds up, where both
-// kernels, each at its best tile and K ranges, were timed (µs a replayed node, fp32 / split):
-// 512×768×768 17.5 / 18.8, 512×3072×768 (1.2e9) 33.5 / 33.0, 256×2560×2560 (1.7e9) 41.6 /
-// 35.8, 1024×2304×768 47.7 / 39.0, 4096×1024×1024 76 / 62, 1024×2560×4096 195 / 120.
+// The family of a GEMM: the split-bf16 kernel from 1.5e9 multiply-adds up.  Both kernels on
+// the tile and K ranges that choose_dma gives them, µs a replayed node, fp32 / split:
+// 666×2304×768 (1.2e9) 34.8 / 33.0, 768×2304×768 (1.4e9) 35.0 / 32.9, 256×2560×2560 (1.7e9)
+// 41.0 / 36.6, 2048×1024×1024 44.2 / 42.6, 1024×4096×512 44.6 / 41.6, 1024×768×3072 (2.4e9)
+// 49.3 / 44.8, 1536×2304×768 58.0 / 49.1, 4096×1024×1024 74 / 64, 512×2560×2560 66 / 54.  A
+// size where a measured fp32 tile is faster than that stays with it (lbr_tuned_fp32_size).
 // Below, a tile's few K steps are a chain of load, split and MFMA latencies on either
 // kernel, and the norm prologue and the one-kernel MLP (fp32) cover the smallest.
 // LBR_GEMM_SPLIT=0 keeps the fp32 kernel, =1 takes the split wherever its operands allow; a
@@ -1141,6 +1143,7 @@ Family gemm_family(long long M, long long N, int K, long long batches) {
     std::string name;
     if (getenv("LBR_GEMM_TILE")) return forced_tile(&name);
     if (const char* e = getenv("LBR_GEMM_SPLIT")) return atoi(e) != 0 ? SPLIT : FP32;
+    if (batches == 1 && lbr_tuned_fp32_size(M, N, K)) return FP32;
     return (double)M * (double)N * (double)K * (double)batches > 1.5e9 ? SPLIT : FP32;
 }
 

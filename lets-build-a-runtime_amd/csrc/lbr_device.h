@@ -421,6 +421,8 @@ bool gemm_dma_tile_pairs(int tile);
 bool gemm_dma_split2(Step* s);
 bool gemm_dma_retile(Step* s, int tile);
 bool gemm_dma_set_ksplit(Step* s, int ks);
+// Whether the measured tiles keep every GEMM of this size on the fp32 kernel (executor.hip).
+bool lbr_tuned_fp32_size(long long M, long long N, long long K);
 // Index of the DMA tile called `name` ("32x48", "64x64" ...) in the step's family (fp32 or
 // split-bf16), or -1.
 int gemm_dma_tile_by_name(const Step& s, const char* name);

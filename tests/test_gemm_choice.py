@@ -39,3 +39,30 @@ def test_ragged_k_with_ranges_it_gives(monkeypatch, K, ks):
     monkeypatch.setenv("LBR_GEMM_KSPLIT", str(ks))
     name, tile, split, got = _choice(300, 70, K)
     assert name == "gemm_mfma_f32_nt" and tile and split and got == ks
+
+
+@pytest.mark.parametrize("M,N,K,batches,split", [
+    (512, 3072, 768, 1, False), (1023, 1909, 768, 1, False), (1024, 1909, 768, 1, True), (2, 1 << 13, 1 << 13, 12, True),
+    (1024, 2304, 768, 1, False),   # measured: an fp32 tile is faster
+    (1024, 2304, 768, 2, True), (1024, 3072, 768, 1, True), (1024, 768, 3072, 1, True)])
+def test_family_of_a_gemm(monkeypatch, M, N, K, batches, split):
+    """Above 1.5e9 multiply-adds the split-bf16 kernel, but for sizes measured to be faster without."""
+    name, tile, got, _ = _choice(M, N, K, batches)
+    assert (name, got) == ("gemm_dma_f32_nt", split) and tile
+    for force in (0, 1):
+        monkeypatch.setenv("LBR_GEMM_SPLIT", str(force))
+        assert _choice(M, N, K, batches)[2] == bool(force)
+
+
+@pytest.mark.parametrize("K,force,split", [(200, None, True), (4, None, True), (200, "1", True), (200, "0", False),
+                                           (202, None, False), (202, "1", False)])
+def test_family_of_a_ragged_k(monkeypatch, K, force, split):
+    """A K that is a multiple of 4 but not of 32 takes the split kernel at any size unless that is
+    switched off; one that is no multiple of 4 has the register-staged kernel alone."""
+    if force is not None:
+        monkeypatch.setenv("LBR_GEMM_SPLIT", force)
+    assert _choice(30, 70, K)[::2] == ("gemm_mfma_f32_nt", split)
+
+
+def test_transposed_b_only():
+    assert not _choice(2048, 2048, 2048, trans_b=0)[2]
