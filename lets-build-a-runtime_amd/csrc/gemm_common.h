@@ -317,21 +317,30 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, float* lds, con
         }
         return;
     }
+    // One loop for GELU, so that its elements' chains overlap, and one for the rest (GELU MLP layer
+    // of 512 tokens and width 768: 59.85 µs, against 60.3 with the choice made element by element).
+    auto store = [&](auto f) {
 #pragma unroll
-    for (int j = 0; j < CG; ++j) {
-        const int n = nw + j * CB + cl;
-        if (n >= N) continue;
-        const float bv = HAS_BIAS ? bias[n] : 0.f;
+        for (int j = 0; j < CG; ++j) {
+            const int n = nw + j * CB + cl;
+            if (n >= N) continue;
+            const float bv = HAS_BIAS ? bias[n] : 0.f;
 #pragma unroll
-        for (int i = 0; i < RG; ++i)
+            for (int i = 0; i < RG; ++i) {
+                float v[4];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int m = mw + i * RS + r;
-                if (m >= M) continue;
-                const float v = HAS_BIAS ? (acc_at(acc, i, j, r) + bv) : alpha * acc_at(acc, i, j, r);
-                C[(long long)m * N + n] = lbr_act(act, v);
+                for (int r = 0; r < 4; ++r)
+                    v[r] = f(HAS_BIAS ? (acc_at(acc, i, j, r) + bv) : alpha * acc_at(acc, i, j, r));
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int m = mw + i * RS + r;
+                    if (m < M) C[(long long)m * N + n] = v[r];
+                }
             }
-    }
+        }
+    };
+    if (act == LBR_ACT_GELU) store([](float v) { return lbr_gelu_tanh(v); });
+    else store([act](float v) { return lbr_act(act, v); });
 }
 
 // Kernel arguments of a decoded or fused GEMM step, and its split-K reduction (gemm.hip).
