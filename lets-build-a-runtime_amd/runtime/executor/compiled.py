@@ -266,20 +266,21 @@ class CompiledExecutor(Executor):
         """Every kernel step of the compiled plan: its kernel (and full step name, with the
         fused parts), the nodes it covers, and the schedule its launch arguments encode
         (attention: causal fold, key-range split workgroups, deferred output, key-quartered
-        16-row kernel and whether it reads K fragment-major; GEMM: DMA tile
-        index, K ranges, norm prologue, norm in the split-K reduce and whether the split was
+        16-row kernel and whether it reads K fragment-major; GEMM: its tile ("legacy": the
+        register-staged kernel) and whether that is the split-bf16 kernel's, DMA tile index
+        (-1 for a K that is no multiple of 32), K ranges, norm prologue, norm in the split-K reduce and whether the split was
         made for it, head splits it stores fragment-major (bit mask), head-prologue parts
         its epilogue applies; head prologue: float4 kernel or one wavefront per row, and
         how many Q/K parts one launch covers)."""
         lib, h = self._lib, self._plan_handle
         first, count, kind = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
-        ints = (ctypes.c_longlong * 40)()
+        ints = (ctypes.c_longlong * 41)()
         names = self.kernel_names()
         out = []
         for st in range(lib.lbr_plan_num_steps(h)):
             lib.check(lib.lbr_plan_step_info(h, st, ctypes.byref(first), ctypes.byref(count), ctypes.byref(kind)),
                       "lbr_plan_step_info")
-            lib.check(lib.lbr_plan_step_args(h, st, ints, 40), "lbr_plan_step_args")
+            lib.check(lib.lbr_plan_step_args(h, st, ints, 41), "lbr_plan_step_args")
             d = {"kernel": names[first.value].split("+")[0], "name": names[first.value], "first": first.value,
                  "count": count.value, "kind": FUSE_KINDS.get(kind.value, "?")}
             if d["kernel"].startswith(("attn_fwd_mfma16", "attn_fwd_kq")):
@@ -287,10 +288,11 @@ class CompiledExecutor(Executor):
                          k_frag=bool(ints[15]) and bool(ints[16]),
                          block_rows=16 if ints[15] else 64 if ints[18] else 128)
             elif d["kernel"].startswith("gemm_"):
+                tile = int(ints[40] or ints[14]) - 1   # [40]: split-bf16 tile of a ragged K
                 d.update(m=int(ints[0]), n=int(ints[1]), k=int(ints[2]),
-                         tile=lib.lbr_gemm_tile_name(int(ints[14]) - 1).decode() or "legacy",
+                         tile=lib.lbr_gemm_tile_name(tile).decode() or "legacy",
                          ksplit=max(1, int(ints[10])), dma_tile=int(ints[14]) - 1,
-                         split=bool(lib.lbr_gemm_tile_split(int(ints[14]) - 1)), norm=int(ints[15]),
+                         split=bool(lib.lbr_gemm_tile_split(tile)), norm=int(ints[15]),
                          reduce_norm=int(ints[16]), split_for_norm=bool(int(ints[17]) & 256),
                          frag_splits=int(ints[5]) if int(ints[19]) > 0 else 0,
                          head_parts=int(ints[18]))

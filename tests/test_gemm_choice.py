@@ -66,3 +66,14 @@ def test_family_of_a_ragged_k(monkeypatch, K, force, split):
 
 def test_transposed_b_only():
     assert not _choice(2048, 2048, 2048, trans_b=0)[2]
+
+
+@pytest.mark.parametrize("K", [96, 100])
+@pytest.mark.parametrize("tile", ["256x256", "256x128", "128x256", "128x128", "128x64", "64x128", "64x64"])
+def test_forced_tile(monkeypatch, tile, K):
+    """A tile name ending in b3 gives the split kernel's tile, one without the fp32 kernel's."""
+    monkeypatch.setenv("LBR_GEMM_TILE", tile + "b3")
+    assert _choice(300, 70, K)[1:3] == (tile, True)
+    if tile not in ("256x128", "128x256"):   # split tiles alone
+        monkeypatch.setenv("LBR_GEMM_TILE", tile)
+        assert _choice(300, 70, K)[1:3] == ((tile, False) if K % 32 == 0 else ("", False))

@@ -2,8 +2,11 @@
 epilogues, operands of every exponent, and the results it hands to the fp32 matrix cores (infinities,
 NaN, the largest values).
 
-The tolerance is the fp32 kernel's own: a dot product of K terms summed in fp32 is off by at most
-about K·2⁻²⁴ of Σ|a·b|; for the N(0,1) operands here that is below 1e-5 of the largest result."""
+Tolerance: the sum rounds six times per 16 terms and once at the end, each time by less than 2⁻²³ of a
+partial sum and by a random part of it (standard deviation 2⁻²³/√12).  Partial sums stay within three
+times the root of their terms' squares (σ); √n·2⁻²³ of that, for all n roundings, is 3.5 standard
+deviations were every partial sum so large: 2.2e-6 σ at K = 96, 7e-6 at 1036.  A kernel without one of its
+six products would be 1.1e-5 σ or more off (emulated)."""
 
 import numpy as np
 import pytest
@@ -16,6 +19,36 @@ from test_gpu_ops import _gemm_case
 
 pytestmark = pytest.mark.gpu
 
+
+
+def _case(M, N, K, batches, with_bias, tile=None, ks=None, name="gemm_dma_f32_nt"):
+    """A GEMM that has to run on the split kernel, with that tile (None: any) and K ranges."""
+    from runtime.executor.compiled import CompiledExecutor
+    from runtime.planner import plan
+    r = rng(M * 7 + N + K)
+    a, b = randn(r, batches, M, K), randn(r, *((N, K) if batches == 1 else (batches, N, K)))
+    a64, bt64 = a.astype(np.float64), np.swapaxes(b, -2, -1).astype(np.float64)
+    ref, size = a64 @ bt64, 3 * np.sqrt((a64 ** 2) @ (bt64 ** 2)).max()
+    consts, attrs = {"b": b}, {"transpose_b": True}
+    if with_bias:
+        consts["bias"] = randn(r, N)
+        ref, size = ref + consts["bias"], size + np.abs(consts["bias"]).max()
+    else:
+        attrs["alpha"] = 0.3
+        ref, size = ref * np.float32(0.3), size * 0.3
+    g = one_node_graph(OpType.MATMUL_ADD if with_bias else OpType.MATMUL, {"a": a}, (batches, M, N), attrs, consts)
+    ex = CompiledExecutor()
+    ex.compile(plan(g))
+    try:
+        step, = ex.step_params()
+        y = ex.run({"a": a})["out"]
+    finally:
+        ex.close()
+    assert step["name"] == name and step["split"], step
+    assert (tile is None or step["tile"] + "b3" == tile) and (ks is None or step["ksplit"] == ks), step
+    assert np.abs(y - ref).max() <= np.sqrt(6 * -(-K // 16) + 1) * 2.0 ** -23 * size
+
+
 TILES = ["256x256", "256x128", "128x256", "128x128", "128x64", "64x128", "64x64"]
 
 
@@ -25,14 +58,14 @@ TILES = ["256x256", "256x128", "128x256", "128x128", "128x64", "64x128", "64x64"
 def test_split_tiles(monkeypatch, tile, M, N, K, batches, with_bias):
     monkeypatch.setenv("LBR_GEMM_TILE", tile)
     monkeypatch.setenv("LBR_GEMM_KSPLIT", "1")
-    assert _gemm_case(M, N, K, True, batches, batches == 1, with_bias) == "gemm_dma_f32_nt"
+    _case(M, N, K, batches, with_bias, tile, 1)
 
 
 @pytest.mark.parametrize("tile,ks,M,N,K", [("256x256b3", 3, 200, 300, 960), ("64x64b3", 2, 70, 130, 64)])
 def test_split_ksplit(monkeypatch, tile, ks, M, N, K):
     monkeypatch.setenv("LBR_GEMM_TILE", tile)
     monkeypatch.setenv("LBR_GEMM_KSPLIT", str(ks))
-    _gemm_case(M, N, K, True, 1, True, True)
+    _case(M, N, K, 1, True, tile, ks)
 
 
 @pytest.mark.parametrize("tile", ["256x256b3", "128x128b3", "64x128b3"])
@@ -52,7 +85,7 @@ def test_split_ragged_k(monkeypatch, tile, M, N, K, batches):
     if tile:
         monkeypatch.setenv("LBR_GEMM_TILE", tile)
         monkeypatch.setenv("LBR_GEMM_KSPLIT", "1")
-    assert _gemm_case(M, N, K, True, batches, batches == 1, True) == "gemm_mfma_f32_nt"
+    _case(M, N, K, batches, True, tile, 1 if tile else None, "gemm_mfma_f32_nt")
 
 
 @pytest.mark.parametrize("K", [20, 200, 712])
@@ -71,11 +104,17 @@ def _run(a, b):
 
 @pytest.mark.parametrize("tile", ["256x256b3", "64x64b3"])
 def test_split_is_exact_where_fp32_is(monkeypatch, tile):
-    """One term a row: the three planes add up to the fp32 value, to the last bit."""
+    """One term a result.  Times a power of two: each operand's three planes add up to its fp32 value,
+    to the last bit.  Two 12-bit significands (two planes each, and an exact fp32 product): so do the
+    products of their planes."""
     monkeypatch.setenv("LBR_GEMM_TILE", tile)
     monkeypatch.setenv("LBR_GEMM_KSPLIT", "1")
     b = randn(rng(5), 130, 96) * np.exp2(rng(6).integers(-20, 20, (130, 96))).astype(np.float32)
-    np.testing.assert_array_equal(_run(np.eye(96, dtype=np.float32), b), b.T)
+    two = np.exp2(rng(7).integers(-20, 20, 96)).astype(np.float32)
+    np.testing.assert_array_equal(_run(np.diag(two), b), two[:, None] * b.T)
+    np.testing.assert_array_equal(_run(b, np.diag(two)), b * two)
+    d, e = (rng(s).integers(1 << 11, 1 << 12, n).astype(np.float32) for s, n in ((8, 96), (9, (130, 96))))
+    np.testing.assert_array_equal(_run(np.diag(d), -e), -(d[:, None] * e.T))
 
 
 @pytest.mark.parametrize("tile", ["256x256b3", "64x64b3"])
