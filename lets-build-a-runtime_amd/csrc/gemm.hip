@@ -1041,7 +1041,8 @@ constexpr DmaTile kDmaTiles[] = {
     {32, 96, 2, 4, 64, 0.80, "32x96k64", false, false},     // 64 KB LDS
     {64, 64, 2, 4, 64, 0.90, "64x64k64", false, true},      // 64 KB LDS
     // Split-bf16 tiles (gemm_split.hip): efficiency as a multiple of the fp32 peak with
-    // every CU busy (4096×12288×4096: 248, 225, 225, 223, 193, 193, 160 TFLOP/s).
+    // every CU busy (4096×12288×4096: 248, 225, 225, 223, 193, 193, 160 TFLOP/s on the box of the
+    // fit; another, at a lower power limit, ran the first six at 238, 217, 218, 206, 180, 180).
     {256, 256, 1, 8, 32, 1.58, "256x256", true, true, SPLIT, 0, 1.50},
     {256, 128, 1, 8, 32, 1.43, "256x128", true, true, SPLIT, 1, 0.86},
     {128, 256, 1, 8, 32, 1.43, "128x256", true, true, SPLIT, 2, 0.86},
@@ -1481,9 +1482,9 @@ int decode_matmul(const OpNode* n, Step* s) {
     }
     // B [N, K] with K a multiple of 4 but not of 32, whole 16-byte rows: the split kernel
     // with its columns past K read as zero, at any size; it has a tile for small grids where
-    // the register-staged kernel has 128×128 alone (µs, split against register-staged:
-    // 231×600×200 9.9 / 20.1, 231×200×712 11.3 / 55, 5×30×20 4.2 / 5.0, 3×1000×4100 15.6 / 30,
-    // 1000×4100×2564 145 / 260).  The step keeps the
+    // the register-staged kernel has 128×128 alone (µs in a kernel trace, K ranges' sum included, split
+    // against register-staged: 231×600×200 8.8 / 25.8, 231×200×712 12.7 / 60.6, 5×30×20 3.9 / 5.1,
+    // 3×1000×4100 16.3 / 30.2, 1000×4100×2564 147 / 256).  The step keeps the
     // register-staged kernel's name and epilogues (residual, head scatter).  Overrides that no
     // split tile meets (a K range count that K does not give, an unknown tile name) leave the
     // GEMM to the register-staged kernel.

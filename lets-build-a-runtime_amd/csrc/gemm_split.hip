@@ -1,15 +1,17 @@
 // gemm_split.hip — the fp32 GEMM C = A · Bᵀ on the bf16 matrix cores.
 //
 // An fp32 value is the exact sum of three bf16 values (8 + 8 + 8 significand bits):
-// h = bf16(x), m = bf16(x − h), l = x − h − m.  A product a·b is then the sum of nine
-// bf16 products, each exact in the MFMA's fp32 accumulator input; the six with a weight of
-// at least 2⁻¹⁶ are taken and the three below (m·l, l·m, l·l, together at most 2⁻²³ of the
-// product, 2⁻²⁶ on average) are left out.  Six v_mfma_f32_32x32x16_bf16 replace sixteen
-// times their number of v_mfma_f32_16x16x4_f32, at 16 times the rate: 2.67× the fp32
-// matrix peak.  The sum rounds once per 16-wide product instead of once per 4 terms, and
-// the six are added smallest first, so the error against 64 bits is below the fp32
-// kernel's at every K (N(0,1) rows: 1.1e-7 / 4.2e-7 / 9.8e-7 at K = 64 / 768 / 4096 against
-// 1.4e-7 / 5.0e-7 / 1.15e-6; GELU outputs at K = 16384: 1.8e-6 against 2.3e-6).
+// h = bf16(x), m = bf16(x − h), l = x − h − m (the splitting of a float into an unevaluated
+// sum of shorter ones, Dekker 1971).  A product a·b is then the sum of nine bf16 products,
+// each exact in the MFMA's fp32 accumulator input; the six largest are taken and m·l, l·m and
+// l·l left out, together at most 2⁻²⁴ of the product (0.09·2⁻²⁴ rms over 2·10⁶ pairs).  Six
+// v_mfma_f32_32x32x16_bf16 replace sixteen v_mfma_f32_16x16x4_f32 in 6/16 of their time: 2.67×
+// the fp32 matrix peak.  The sum rounds six times per 16 terms, smallest products first, the
+// fp32 kernel's four times.  Measured, root mean square error against 64 bits in the results'
+// rms, N(0,1) rows of K = 4 / 20 / 64 / 256 / 768 / 4096 / 16384: 3.2e-8 / 6.3e-8 / 1.1e-7 / 2.4e-7 /
+// 2.4e-7 / 2.7e-7 / 5.3e-7 against the fp32 kernels' 4.1e-8 / 8.2e-8 / 1.4e-7 / 2.9e-7 / 2.9e-7 /
+// 4.4e-7 / 6.2e-7, each on its own tile and K ranges; lower at all 16 values of K tried, and
+// with GELU outputs for A too.
 //
 // Range: both operands are taken times 2²⁴ and the sum times 2⁻⁴⁸, all exact, so that the
 // planes of every finite value below 2¹⁰⁴, subnormals included, are zero or normal bf16
@@ -33,10 +35,10 @@
 // of a wavefront hit every bank once (SQ_LDS_BANK_CONFLICT 0; row-major planes of 32 bytes
 // a row had two conflict cycles a read and cost 2%).
 //
-// What bounds it: 4096×12288×4096 takes 1723 µs, 239 TFLOP/s (1.44 PFLOP/s of bf16
-// products), against 2790 µs and 148 for the fp32 kernel; MFMAs alone, on such data, run at
-// 295, the power limit (torch's bf16 mm on 8192³: 1.31 PFLOP/s).  Splitting costs 10% of
-// that and the loads the rest.
+// What bounds it: 4096×12288×4096 takes 1731 µs, 238 TFLOP/s (1.43 PFLOP/s of bf16
+// products), against 2765 µs and 149 for the fp32 kernel; MFMAs alone, on such data, run at
+// 295, the power limit (a library's bf16 product of 8192³: 1.28-1.37 PFLOP/s over boxes, which
+// differ by up to 8%).  Splitting costs 10% of that and the loads the rest.
 #include "gemm_common.h"
 
 #include <type_traits>
