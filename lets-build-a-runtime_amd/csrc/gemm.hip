@@ -1041,7 +1041,7 @@ constexpr DmaTile kDmaTiles[] = {
     {32, 96, 2, 4, 64, 0.80, "32x96k64", false, false},     // 64 KB LDS
     {64, 64, 2, 4, 64, 0.90, "64x64k64", false, true},      // 64 KB LDS
     // Split-bf16 tiles (gemm_split.hip): efficiency as a multiple of the fp32 peak with
-    // every CU busy (4096×12288×4096: 248, 225, 225, 223, 193, 193, 160 TFLOP/s on the box of the
+    // every CU busy (4096×12288×4096: 248, 225, 225, 223, 193, 193, 160 TFLOP/s on the card of the
     // fit; another, at a lower power limit, ran the first six at 238, 217, 218, 206, 180, 180).
     {256, 256, 1, 8, 32, 1.58, "256x256", true, true, SPLIT, 0, 1.50},
     {256, 128, 1, 8, 32, 1.43, "256x128", true, true, SPLIT, 1, 0.86},

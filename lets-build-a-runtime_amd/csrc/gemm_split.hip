@@ -37,7 +37,7 @@
 //
 // What bounds it: 4096×12288×4096 takes 1731 µs, 238 TFLOP/s (1.43 PFLOP/s of bf16
 // products), against 2765 µs and 149 for the fp32 kernel; MFMAs alone, on such data, run at
-// 295, the power limit (a library's bf16 product of 8192³: 1.28-1.37 PFLOP/s over boxes, which
+// 295, the power limit (a library's bf16 product of 8192³: 1.28-1.37 PFLOP/s over cards, which
 // differ by up to 8%).  Splitting costs 10% of that and the loads the rest.
 #include "gemm_common.h"
 
